@@ -180,8 +180,9 @@ def _inputs(case: dict, seed: int) -> dict:
     raise ValueError(kind)
 
 
-def _captured(call):
-    """The program's step captured once; returns its replay and its outputs."""
+def _captured(call) -> dict:
+    """The program's step captured once: its replay, its outputs, and the step
+    itself, whose plans own the workspaces that the replay uses."""
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
@@ -191,7 +192,7 @@ def _captured(call):
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         out = call()
-    return graph, out
+    return {"call": call, "graph": graph, "out": out}
 
 
 def _decode_plan(case: dict, seed: int):
@@ -226,7 +227,7 @@ def prepare(case: dict, seed: int):
             act = gu(s["x"], s["y"], s["norm"], xout, s["wgu"])
             return {"xout": xout, "act": act, "y": down(act, s["wd"])}
 
-        s["graph"], s["out"] = _captured(call)
+        s.update(_captured(call))
     elif kind == "o_proj":
         s["mm"] = K.pick_matmul(s["a"], s["wo"])
     elif kind == "head_topk":
@@ -238,7 +239,7 @@ def prepare(case: dict, seed: int):
             vals, idxs = K.fast_topk(logits, case["k"])
             return {"xout": xout, "logits": logits, "vals": vals, "idxs": idxs}
 
-        s["graph"], s["out"] = _captured(call)
+        s.update(_captured(call))
     elif kind == "head_argmax":
         mm = K.pick_lm_argmax(s["x"], s["lm_head"], EPS)
         xout = torch.empty_like(s["x"])
@@ -247,7 +248,7 @@ def prepare(case: dict, seed: int):
             ids, maxv = mm(s["x"], s["y"], s["norm"], xout, s["lm_head"])
             return {"xout": xout, "ids": ids, "maxv": maxv}
 
-        s["graph"], s["out"] = _captured(call)
+        s.update(_captured(call))
     elif kind in ("attention", "attn_half"):
         B, R, cap = case["B"], case["R"], case["cap"]
         attn = K.pick_attention(B, HQ, HKV, HD, cap, case["ctx"], DEV, R=R, tree=R > 1, maxlen=cap)
@@ -271,7 +272,7 @@ def prepare(case: dict, seed: int):
                 o = mm_o(attn_out.view(B * R, HQ * HD), s["wo"])
                 return {"xout": xout, "out": attn_out, "o": o, "k_cache": s["k_cache"], "v_cache": s["v_cache"]}
 
-        s["graph"], s["out"] = _captured(call)
+        s.update(_captured(call))
     elif kind == "prefill_rows":
         B, T, cap = case["B"], case["T"], s["cap"]
         s["pos"] = torch.zeros((B,), dtype=torch.int32, device=DEV)
