@@ -21,7 +21,8 @@
  * and the data pointers may then be NULL.
  *
  * Workspace: ops that need device scratch take (ws, ws_bytes); query the size
- * with sk_workspace_bytes() for the same op/shape/config and allocate it once,
+ * with sk_workspace_bytes() (or sk_workspace_bytes_preferred(), for the fastest
+ * plan of calls without a config) for the same op/shape/config and allocate it once,
  * zero-filled (outside graph capture).  Its first bytes hold arrival counters
  * that let the last workgroup of a tile finish a split-K sum or an argmax in
  * the same kernel; every call leaves them at zero again, so the workspace is
@@ -77,7 +78,8 @@ typedef enum sk_path {
   SK_PATH_MFMA = 1,       /* v_mfma_f32_16x16x32_bf16 tiles, 16 weight rows per wave tile */
   SK_PATH_GEMV = 2,       /* VALU v_dot2_f32_bf16, lanes span K, DPP/shuffle lane reduction */
   SK_PATH_MFMA_LDS = 3,   /* MFMA fed from LDS: weight rows loaded 1 KiB-contiguous, transposed in LDS */
-  SK_PATH_WIDE = 4        /* up to 128 rows per workgroup: weight tile staged once in LDS for all rows */
+  SK_PATH_WIDE = 4,       /* up to 128 rows per workgroup: weight tile staged once in LDS for all rows */
+  SK_PATH_STREAM = 5      /* up to 128 rows per workgroup: both operands loaded straight into LDS rings */
 } sk_path;
 
 /*
@@ -86,7 +88,8 @@ typedef enum sk_path {
  * from an offline-tuned table (sk_default_config) and an explicit config can
  * be passed to any op (NULL = default) to test or time one candidate.
  *
- *   path   : SK_PATH_MFMA, SK_PATH_MFMA_LDS or SK_PATH_GEMV
+ *   path   : SK_PATH_MFMA, SK_PATH_MFMA_LDS, SK_PATH_GEMV, SK_PATH_WIDE or
+ *            SK_PATH_STREAM
  *   waves  : wavefronts per workgroup; they split the workgroup's K slice and
  *            their fp32 partials are summed in LDS in fixed wave order
  *   ku     : K units per wave (MFMA: 32 columns; GEMV: 512 columns; WIDE: 8,
@@ -126,6 +129,14 @@ typedef enum sk_path {
  *            that stages the activation rows in LDS beside the weight tile
  *            (128-column steps; four waves of 32 activation rows, or eight
  *            whose pairs split each step's K columns).
+ *
+ *            SK_PATH_STREAM reads it as the waves that share one K group's
+ *            rows (waves = K groups x groups; 4 x 1 up to 16 rows, 2 x 2 up
+ *            to 64, 1 x 4 with ku 4 up to 128).  There ku is 2 or 4 (units of
+ *            64 or 128 columns; K a multiple of the unit), rows the output
+ *            columns per tile (up to 80, gate/up up to 40), grid 0 (one
+ *            workgroup per tile and split); no fused argmax, gate/up with one
+ *            split, of the hand-off ops the producer (rows a multiple of 16).
  *
  * Rows per launch: at most 64 without row groups; with a configuration that
  * splits them into groups (compiled for groups of up to 32 rows), up to 128
@@ -167,6 +178,14 @@ int sk_check_config(int op, int M, int N, int K, const sk_config* cfg);
 
 /* Workspace bytes op needs at (M, N, K) with cfg (NULL = default config). */
 size_t sk_workspace_bytes(int op, int M, int N, int K, const sk_config* cfg);
+
+/* Workspace bytes with which a call without a configuration runs its fastest
+ * plan.  Such a call takes the stream path (SK_PATH_STREAM) at the shapes and
+ * row counts where that measured faster than sk_default_config's plan and its
+ * workspace fits ws_bytes; where the fastest plan splits K, this is more than
+ * sk_workspace_bytes, which is the least that any call needs.  Zero-filled
+ * once like every workspace; the plan depends only on op, shape and ws_bytes. */
+size_t sk_workspace_bytes_preferred(int op, int M, int N, int K);
 
 /* C[M,N] = bf16(A[M,K] @ W[N,K]^T), fp32 accumulation.
  * Replaces SkinnyMatmul.__call__ / _skinny_kernel + _sum_kernel

@@ -44,10 +44,12 @@ SK_PATH_MFMA = 1
 SK_PATH_GEMV = 2
 SK_PATH_MFMA_LDS = 3
 SK_PATH_WIDE = 4
+SK_PATH_STREAM = 5
 
 # Every symbol include/starter_amd.h declares (checked by the CPU tests).
 EXPORTS = (
     "sk_version", "sk_strerror", "sk_default_config", "sk_check_config", "sk_workspace_bytes",
+    "sk_workspace_bytes_preferred",
     "sk_gemm_bf16", "sk_gemm_bf16_noalloc", "sk_gateup_swiglu_bf16", "sk_lm_argmax_bf16", "sk_argmax_bf16",
     "sk_add_rmsnorm_bf16", "sk_swiglu_bf16",
     "sk_rmsnorm_gemm_bf16", "sk_rmsnorm_gateup_swiglu_bf16", "sk_rmsnorm_lm_argmax_bf16",
@@ -106,6 +108,7 @@ _SIGNATURES = {
     "sk_default_config": (_i32, [_i32, _i32, _i32, _i32, _i32, _cfgp]),
     "sk_check_config": (_i32, [_i32, _i32, _i32, _i32, _cfgp]),
     "sk_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _cfgp]),
+    "sk_workspace_bytes_preferred": (_sz, [_i32, _i32, _i32, _i32]),
     "sk_gemm_bf16": (_i32, [_p, _i64, _p, _i64, _p, _i64, _i32, _i32, _i32, _cfgp, _p, _sz, _p]),
     "sk_gemm_bf16_noalloc": (_i32, [_p, _i64, _p, _i64, _p, _i64, _i32, _i32, _i32, _cfgp, _p]),
     "sk_gateup_swiglu_bf16": (_i32, [_p, _i64, _p, _p, _i64, _p, _i64, _i32, _i32, _i32, _cfgp, _p, _sz, _p]),
@@ -189,3 +192,9 @@ def check_config(op: int, M: int, N: int, K: int, cfg: SkConfig) -> int:
 
 def workspace_bytes(op: int, M: int, N: int, K: int, cfg: SkConfig | None = None) -> int:
     return int(lib().sk_workspace_bytes(op, M, N, K, cfg_ptr(cfg)))
+
+
+def workspace_bytes_preferred(op: int, M: int, N: int, K: int) -> int:
+    """Workspace with which calls without a configuration run their fastest
+    plan (``workspace_bytes`` is the least they run with)."""
+    return int(lib().sk_workspace_bytes_preferred(op, M, N, K))

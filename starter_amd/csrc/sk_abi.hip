@@ -122,6 +122,8 @@ struct Plan {
   int mrows = 0;
   size_t stage_elem = 0;        // LDS bytes per staged tile (0: argmax keeps 8*M bytes)
   size_t lds = 0;               // total dynamic LDS (set once the grid is known)
+  int uc = 0, mg = 0;           // stream path: columns per unit, waves per K group
+  size_t ticket_min = 0;        // least bytes of the workspace's counter area
   bool norm = false;            // the op has the add + RMSNorm prologue
   bool fused = false;           // ... and it runs inside the projection kernel
   sk::KernelFn fn = nullptr;
@@ -130,6 +132,9 @@ struct Plan {
 bool is_norm_op(int op) {
   return op == SK_OP_RMSNORM_GEMM || op == SK_OP_RMSNORM_GATEUP || op == SK_OP_RMSNORM_LM_ARGMAX;
 }
+// Paths that hold every row of a launch in one workgroup (up to kMaxLaunchM
+// rows without row groups); they read `groups` as wave groups.
+bool whole_m_path(int path) { return path == SK_PATH_WIDE || path == SK_PATH_STREAM; }
 // The projection an op performs (the norm ops map to GEMM / GATEUP / LM_ARGMAX).
 int base_op(int op) { return is_norm_op(op) ? op - SK_OP_RMSNORM_GEMM : op; }
 bool is_gemm_family(int op) { return op == SK_OP_GEMM || op == SK_OP_GATEUP || op == SK_OP_LM_ARGMAX; }
@@ -167,6 +172,8 @@ sk::KernelFn plan_kernel(const Plan& pl) {
   if (pl.cfg.path == SK_PATH_MFMA) return sk::mfma_kernel_for(pl.epi, pl.tm, pl.tn, pl.tku);
   if (pl.cfg.path == SK_PATH_WIDE)
     return sk::wide_kernel_for(pl.epi, pl.cfg.waves, pl.cfg.groups > 1 ? pl.cfg.groups : 1, pl.tn);
+  if (pl.cfg.path == SK_PATH_STREAM)
+    return sk::stream_kernel_for(pl.epi, pl.cfg.waves / pl.mg, pl.mg, pl.tm, pl.tn, pl.uc);
   if (pl.cfg.path == SK_PATH_MFMA_LDS)
     return pl.groups > 1 ? sk::mfmt_grouped_kernel_for(pl.epi, pl.tm, pl.tn, pl.tku)
                          : sk::mfmt_kernel_for(pl.epi, pl.tm, pl.tn, pl.tku);
@@ -201,7 +208,7 @@ int plan_shape_impl(int op, int M, int N, int K, const sk_config& c, bool fused,
   // plan is that of one group.
   // (the wide path reads `groups` as the wave groups along the tile's weight
   // slabs, not as row groups)
-  const int groups = c.groups > 1 && c.path != SK_PATH_WIDE ? c.groups : 1;
+  const int groups = c.groups > 1 && !whole_m_path(c.path) ? c.groups : 1;
   if (groups > 1) {
     if (fused || c.path != SK_PATH_MFMA_LDS || (c.ku != 8 && c.ku != 32)) return SK_ERR_CONFIG;
     if (c.grid <= 0 || (c.grid % 8) != 0) return SK_ERR_CONFIG;
@@ -211,7 +218,7 @@ int plan_shape_impl(int op, int M, int N, int K, const sk_config& c, bool fused,
   }
   // more rows than an instance holds: chunked, or row groups (the wide path
   // holds up to kMaxLaunchM rows in one workgroup)
-  if (M > (c.path == SK_PATH_WIDE && groups == 1 ? kMaxLaunchM : kMaxM)) return SK_ERR_SHAPE;
+  if (M > (whole_m_path(c.path) && groups == 1 ? kMaxLaunchM : kMaxM)) return SK_ERR_SHAPE;
   pl->groups = groups;
   pl->mrows = M;
   const bool gateup = (op == SK_OP_GATEUP);
@@ -219,7 +226,11 @@ int plan_shape_impl(int op, int M, int N, int K, const sk_config& c, bool fused,
   if (variant != 0) {
     if (fused) return SK_ERR_CONFIG;
     if (variant == 2 && op != SK_OP_GEMM) return SK_ERR_CONFIG;
-    if (c.path == SK_PATH_WIDE) {
+    if (c.path == SK_PATH_STREAM) {
+      // producers only, in tiles of whole 16-column groups (the finish writes
+      // one partial sum per group)
+      if (variant != 2 || (c.rows & 15) != 0) return SK_ERR_CONFIG;
+    } else if (c.path == SK_PATH_WIDE) {
       // the two-operand wide body: consumers with one K split (whole 16-column
       // groups of partial sums), the producer after split-K partials (its
       // tiles are whole 16-column groups, checked below)
@@ -294,6 +305,22 @@ int plan_shape_impl(int op, int M, int N, int K, const sk_config& c, bool fused,
     pl->tku = sk::kWideChunk;
     partial_rows = 0;
     pl->pre_lds = wn == 4 ? sk::wide2_lds(pl->tn) : sk::wide_weight_lds(pl->tn);
+  } else if (c.path == SK_PATH_STREAM) {
+    // waves = KG * MG, MG = groups; MT and NT follow from the rows.
+    const int mg = c.groups > 1 ? c.groups : 1;
+    const int uc = 32 * c.ku;
+    if ((c.ku != 2 && c.ku != 4) || c.waves % mg != 0 || c.grid != 0 || K % uc != 0) return SK_ERR_CONFIG;
+    if (op == SK_OP_LM_ARGMAX || (gateup && c.split != 1)) return SK_ERR_CONFIG;
+    if (c.rows < 1 || c.rows > 256) return SK_ERR_CONFIG;
+    units = K / uc;
+    pl->uc = uc;
+    pl->mg = mg;
+    pl->tn = cdiv(gateup ? 2 * sk::stream_half(c.rows, uc) : c.rows, 16);
+    pl->tku = uc;
+    for (pl->tm = cdiv(M, 16 * mg); pl->tm <= 8 && !plan_kernel(*pl); ++pl->tm) {}
+    if (pl->tm > 8) return SK_ERR_CONFIG;
+    partial_rows = 0;
+    pl->pre_lds = sk::stream_lds(c.waves / mg, mg, pl->tm, pl->tn, uc);
   } else if (c.path == SK_PATH_GEMV) {
     if (c.rows != 2 && c.rows != 4 && c.rows != 8) return SK_ERR_CONFIG;
     if (M > 8) return SK_ERR_CONFIG;
@@ -312,10 +339,10 @@ int plan_shape_impl(int op, int M, int N, int K, const sk_config& c, bool fused,
   if (!plan_kernel(*pl)) return SK_ERR_CONFIG;
   pl->slice_units = cdiv(units, c.split);
   const long per_wave = c.path == SK_PATH_MFMA_LDS ? 1 : c.ku;
-  // (the wide path's waves all walk the whole slice)
-  if (c.path != SK_PATH_WIDE && (long)c.waves * per_wave < pl->slice_units) return SK_ERR_CONFIG;   // K slice not covered
+  // (the waves of the wide and stream paths walk the whole slice)
+  if (!whole_m_path(c.path) && (long)c.waves * per_wave < pl->slice_units) return SK_ERR_CONFIG;   // K slice not covered
   if (c.split > 1 && (c.split - 1) * pl->slice_units >= units) return SK_ERR_CONFIG;  // empty split
-  const bool lds_fed = c.path == SK_PATH_MFMA_LDS || c.path == SK_PATH_WIDE;
+  const bool lds_fed = c.path == SK_PATH_MFMA_LDS || whole_m_path(c.path);
   const int out_rows = c.path == SK_PATH_MFMA ? (gateup ? 16 : c.rows)
                        : lds_fed             ? (gateup ? 8 * pl->tn : 16 * pl->tn)
                                              : c.rows;
@@ -325,6 +352,10 @@ int plan_shape_impl(int op, int M, int N, int K, const sk_config& c, bool fused,
   if (c.path == SK_PATH_MFMA_LDS) partial_rows = sk::lds_part_stride(pl->tm, pl->tn, pl->tku);
   pl->parts_lds = (size_t)2 * c.waves * M * partial_rows * sizeof(float);
   pl->stage_elem = stage_bytes(pl->epi) * (size_t)M * out_rows;
+  if (c.path == SK_PATH_STREAM) {   // the ring or the epilogue planes, flag included (pre_lds)
+    pl->parts_lds = 0;
+    pl->stage_elem = 0;
+  }
   if (c.path == SK_PATH_WIDE) {   // outputs go straight from registers; the split-K finish's flags
     pl->parts_lds = (size_t)64 * c.waves * sizeof(int);
     pl->stage_elem = 0;
@@ -334,7 +365,7 @@ int plan_shape_impl(int op, int M, int N, int K, const sk_config& c, bool fused,
   pl->lds = plan_lds(*pl, M, tiles_per);
   // The ring path can work with one partial tile buffer (one more barrier per
   // tile) where two would not fit.
-  const bool ring = c.path == SK_PATH_MFMA_LDS && pl->tku != 512;   // (not the wide path)
+  const bool ring = c.path == SK_PATH_MFMA_LDS && pl->tku != 512;   // (not the wide or stream path)
   if (ring && (pl->lds > kMaxLds || (c.grid == 0 && plan_lds(*pl, M, cdiv(pl->nrb, kMaxGrid)) > kMaxLds))) {
     pl->pbuf = 1;
     pl->parts_lds /= 2;
@@ -380,11 +411,15 @@ size_t ticket_bytes(int n) { return (((size_t)n * sizeof(unsigned)) + 255) & ~(s
 // With row groups: one counter (argmax) or one per tile for each group, the
 // argmax candidates of all M rows, and one partials region per group.
 size_t plan_tickets(int op, const Plan& pl) {
-  return ticket_bytes(pl.groups * (base_op(op) == SK_OP_LM_ARGMAX ? 1 : pl.nrb));
+  const size_t n = ticket_bytes(pl.groups * (base_op(op) == SK_OP_LM_ARGMAX ? 1 : pl.nrb));
+  return n > pl.ticket_min ? n : pl.ticket_min;
 }
 size_t plan_workspace(int op, int M, int N, const Plan& pl) {
   op = base_op(op);
   if (op == SK_OP_LM_ARGMAX) return plan_tickets(op, pl) + (size_t)M * sizeof(unsigned long long);
+  if (pl.cfg.split > 1 && pl.cfg.path == SK_PATH_STREAM)   // one block of partials per tile and split
+    return plan_tickets(op, pl) +
+           (size_t)pl.nrb * pl.cfg.split * pl.mrows * sk::stream_part_pitch(pl.tr) * sizeof(float);
   if (pl.cfg.split > 1)
     return plan_tickets(op, pl) +
            (size_t)pl.groups * (op == SK_OP_GATEUP ? 2 : 1) * pl.cfg.split * pl.mrows * (size_t)N * sizeof(float);
@@ -518,6 +553,60 @@ const Tuned kTuned[] = {
     // rows and 193 at 96 (96-row tiles 243 and 229, four row groups 304-342)
     {SK_OP_GEMM, 151936, 2560, 128, {4, 8, 8, 128, 1, 0, 4}},
 };
+
+// Stream-path plans (sk_stream.hpp) of calls without an explicit
+// configuration, by shape and row range; the first entry whose workspace fits
+// what the caller gave is taken, else the table above applies.  Measured like
+// the table above on one MI355X; "was" is that table's plan in the same run.
+//  * The tile height gives every CU one tile (N * split / 256 rows, whole
+//    16-row slabs where that costs no CU): a workgroup fills a CU's LDS.
+//  * Splits: down and o_proj have too few rows for one tile per CU, and
+//    splitting K instead of using 10-row tiles cuts the activation bytes each
+//    CU reads; at 32 rows and more that outweighs the finish's round trips
+//    (about 2.5 us).  Their least workspace (sk_workspace_bytes) allows three
+//    splits of 32-row tiles or none; sk_workspace_bytes_preferred covers the
+//    first entry.
+//  * qkv and o_proj up to 16 rows and gate_up up to 16 stay on the ring path
+//    where that measured within 2%; qkv at 49-64 rows runs 128-column units
+//    (13.4 us with 64-column ones).
+struct StreamEntry {
+  int op, N, K, m_lo, m_hi;
+  sk_config cfg;   // {path, waves, ku = unit columns / 32, tile rows, split, 0, waves per K group}
+};
+
+const StreamEntry kStream[] = {
+    {SK_OP_GATEUP, 9728, 2560, 17, 64, {5, 4, 2, 38, 1, 0, 2}},     // gate_up 32 rows 20.9 us (was 21.3), 64 24.5 (28.0)
+    {SK_OP_GATEUP, 9728, 2560, 65, 128, {5, 4, 4, 40, 1, 0, 4}},    // gate_up 96 rows 26.4 (30.4), 128 27.9 (35.2)
+    {SK_OP_GEMM, 6144, 2560, 2, 16, {5, 4, 2, 24, 1, 0, 1}},        // qkv 8 rows 7.7 (8.2), 16 8.2 (8.7)
+    {SK_OP_GEMM, 6144, 2560, 17, 48, {5, 4, 2, 24, 1, 0, 2}},       // qkv 32 rows 9.6 (10.2), 40 10.7 (11.7)
+    {SK_OP_GEMM, 6144, 2560, 49, 64, {5, 4, 4, 24, 1, 0, 2}},       // qkv 49 rows 11.5 (11.6), 64 12.0 (12.1)
+    {SK_OP_GEMM, 6144, 2560, 65, 128, {5, 4, 4, 24, 1, 0, 4}},      // qkv 96 rows 16.0 (16.6), 128 16.8 (17.7)
+    {SK_OP_GEMM, 2560, 4096, 17, 64, {5, 4, 2, 32, 3, 0, 2}},       // o_proj 32 rows 8.8 (9.5), 64 10.8 (12.7)
+    {SK_OP_GEMM, 2560, 4096, 97, 128, {5, 4, 4, 32, 3, 0, 4}},      // o_proj 128 rows 14.2 (17.3)
+    {SK_OP_GEMM, 2560, 9728, 3, 16, {5, 4, 2, 32, 3, 0, 1}},        // down 8 rows 12.0 (13.8), 16 12.7 (15.3)
+    {SK_OP_GEMM, 2560, 9728, 17, 64, {5, 4, 2, 40, 4, 0, 2}},       // down 32 rows 14.3 (17.7), 64 19.2 (21.9)
+    {SK_OP_GEMM, 2560, 9728, 17, 64, {5, 4, 2, 32, 3, 0, 2}},       // down 32 rows 14.9, 64 20.1
+    {SK_OP_GEMM, 2560, 9728, 65, 128, {5, 4, 4, 40, 4, 0, 4}},      // down 96 rows 21.7 (24.3), 128 23.2 (27.6)
+    {SK_OP_GEMM, 2560, 9728, 65, 128, {5, 4, 4, 32, 3, 0, 4}},      // down 96 rows 22.5, 128 24.5
+    // residual producers (tiles of whole 16-column groups)
+    {SK_OP_RESID_GEMM, 2560, 4096, 17, 64, {5, 4, 2, 32, 3, 0, 2}},     // o_proj 32 rows 9.8 (10.1), 64 12.5 (14.0)
+    {SK_OP_RESID_GEMM, 2560, 4096, 97, 128, {5, 4, 4, 32, 3, 0, 4}},    // o_proj 128 rows 17.9 (20.7)
+    {SK_OP_RESID_GEMM, 2560, 9728, 3, 16, {5, 4, 2, 32, 3, 0, 1}},      // down 8 rows 12.9 (14.8), 16 13.3 (15.2)
+    {SK_OP_RESID_GEMM, 2560, 9728, 17, 64, {5, 4, 2, 32, 3, 0, 2}},     // down 32 rows 15.7 (20.0), 64 21.1 (28.2)
+    {SK_OP_RESID_GEMM, 2560, 9728, 65, 128, {5, 4, 4, 32, 3, 0, 4}},    // down 96 rows 24.8 (27.5), 128 27.7 (31.4)
+};
+
+// The n-th stream entry of op/N/K at M rows, or nullptr.
+const StreamEntry* stream_lookup(int op, int M, int N, int K, int n) {
+  for (const StreamEntry& e : kStream)
+    if (e.op == op && e.N == N && e.K == K && e.m_lo <= M && M <= e.m_hi && n-- == 0) return &e;
+  return nullptr;
+}
+
+// The stream kernels address a tile's rows with 32-bit byte offsets.
+bool stream_strides_ok(int M, int64_t lda, int rows, int64_t ldw) {
+  return M * lda * 2 < 0x7F000000ll && rows * ldw * 2 < 0x7F000000ll;
+}
 
 // Tuned entry for op/N/K at the smallest tuned row count >= M among op's own
 // entries and those of `also` (-1: none), op's own entry first at equal row
@@ -687,7 +776,9 @@ int bind_plan(Plan* pl, int num_cu, int* grid) {
   if (threads > fi.max_threads) return SK_ERR_CONFIG;
   pl->fn = fn;
   const int S = pl->cfg.split;
-  if (pl->cfg.grid > 0) {
+  if (pl->cfg.path == SK_PATH_STREAM) {   // one workgroup per tile and split
+    *grid = pl->nrb * S;
+  } else if (pl->cfg.grid > 0) {
     *grid = pl->cfg.grid;
   } else {
     // Resident workgroups per K split from the occupancy at one staged tile,
@@ -786,7 +877,7 @@ int launch_rows(int op, int M, int N, int K, const sk_config* cfg) {
   const int R = M < kMaxLaunchM ? M : kMaxLaunchM;
   sk_config c;
   Plan pl;
-  if (resolve_config(op, R, N, K, cfg, &c) == SK_OK && (c.groups > 1 || c.path == SK_PATH_WIDE) &&
+  if (resolve_config(op, R, N, K, cfg, &c) == SK_OK && (c.groups > 1 || whole_m_path(c.path)) &&
       plan_shape(op, R, N, K, c, &pl) == SK_OK)
     return kMaxLaunchM;
   return kMaxM;
@@ -807,7 +898,7 @@ int plan_call(int op, int M, int N, int K, const sk_config* cfg, CallPlan* cp) {
     // 128-row launches, e.g. one row of 129) runs with as many groups as
     // hold a row, so the configuration default_config returns for the whole
     // call is accepted for every launch.
-    if (cp->nplans == 2 && i == 1 && c.groups > 1 && c.path != SK_PATH_WIDE) {
+    if (cp->nplans == 2 && i == 1 && c.groups > 1 && !whole_m_path(c.path)) {
       const int rows = cp->chunk_rows[i];
       int g = c.groups;
       while (g > 1 && (g - 1) * cdiv(rows, g) >= rows) --g;
@@ -836,6 +927,37 @@ int plan_call(int op, int M, int N, int K, const sk_config* cfg, CallPlan* cp) {
     cp->need = cp->norm_off + (size_t)M * K * sizeof(sk_bf16);
   }
   return SK_OK;
+}
+
+// The call with stream-path plans in place of cp's, taking the n-th entry of
+// each launch's rows where there is one; false when no launch has an n-th
+// entry.  The counters of both plans lie inside one area, so calls with and
+// without a configuration can share a workspace.
+bool stream_call(int op, int M, int N, int K, const CallPlan& cp, int n, CallPlan* out) {
+  if (cp.fused) return false;
+  const int bop = base_op(op);
+  *out = cp;
+  bool any = false;
+  out->base_need = 0;
+  for (int i = 0; i < cp.nplans; ++i) {
+    if (const StreamEntry* e = stream_lookup(bop, cp.chunk_rows[i], N, K, n)) {
+      Plan pl;
+      if (plan_shape_impl(bop, cp.chunk_rows[i], N, K, e->cfg, false, &pl) == SK_OK) {
+        if (cp.plans[i].cfg.split > 1) pl.ticket_min = plan_tickets(bop, cp.plans[i]);
+        pl.norm = cp.plans[i].norm;
+        out->plans[i] = pl;
+        any = true;
+      }
+    }
+    const size_t need = plan_workspace(bop, cp.chunk_rows[i], N, out->plans[i]);
+    if (need > out->base_need) out->base_need = need;
+  }
+  out->need = out->base_need;
+  if (is_norm_op(op)) {
+    out->norm_off = align256(out->base_need);
+    out->need = out->norm_off + (size_t)M * K * sizeof(sk_bf16);
+  }
+  return any;
 }
 
 // Shared driver of the GEMM-family ops.  nrm != nullptr: A is x and the
@@ -872,6 +994,18 @@ int run_gemm_family(int op, const sk_bf16* A, int64_t lda, const NormIn* nrm, co
     if (cp.need > SK_NOALLOC_SCRATCH_BYTES) return SK_ERR_SCRATCH;
   } else if (cp.need > 0 && (!ws || ws_bytes < cp.need)) {
     return SK_ERR_WORKSPACE;
+  }
+  if (!cfg || cfg->path == SK_PATH_AUTO) {
+    // (the allocation-free call takes the plan that the least workspace gets)
+    const size_t avail = noalloc ? cp.need : (ws ? ws_bytes : 0);
+    CallPlan alt;
+    for (int n = 0; stream_call(op, M, N, K, cp, n, &alt); ++n) {
+      if (alt.need > avail) continue;
+      if (stream_strides_ok(M, nrm ? K : lda, 256, ldw)) cp = alt;
+      break;
+    }
+  } else if (cfg->path == SK_PATH_STREAM && !stream_strides_ok(M, nrm ? K : lda, 256, ldw)) {
+    return SK_ERR_SHAPE;
   }
   int num_cu = 0;
   st = device_info(&num_cu);
@@ -1027,6 +1161,14 @@ int plan_handoff(int op, int M, int N, int K, const sk_config* cfg, Plan* pl) {
   return plan_shape_impl(handoff_base(op), M, N, K, c, false, pl, handoff_variant(op));
 }
 
+// The n-th stream plan of a hand-off op in place of pl (its default plan).
+bool stream_handoff(int op, int M, int N, int K, const Plan& def, int n, Plan* pl) {
+  const StreamEntry* e = stream_lookup(op, M, N, K, n);
+  if (!e || plan_shape_impl(handoff_base(op), M, N, K, e->cfg, false, pl, handoff_variant(op)) != SK_OK) return false;
+  if (def.cfg.split > 1) pl->ticket_min = plan_tickets(handoff_base(op), def);
+  return true;
+}
+
 size_t handoff_workspace(int op, int M, int N, int K, const sk_config* cfg) {
   Plan pl;
   if (plan_handoff(op, M, N, K, cfg, &pl)) return 0;
@@ -1078,6 +1220,16 @@ int run_handoff(int op, const sk_bf16* A, int64_t lda, const Handoff& h, const s
   if (st) return st;
   const size_t need = plan_workspace(bop, M, N, pl);
   if (need > 0 && (!ws || ws_bytes < need)) return SK_ERR_WORKSPACE;
+  if (!cfg || cfg->path == SK_PATH_AUTO) {
+    Plan alt;
+    for (int n = 0; stream_handoff(op, M, N, K, pl, n, &alt); ++n) {
+      if (plan_workspace(bop, M, N, alt) > (ws ? ws_bytes : 0)) continue;
+      if (stream_strides_ok(M, lda, 256, ldw)) pl = alt;
+      break;
+    }
+  } else if (cfg->path == SK_PATH_STREAM && !stream_strides_ok(M, lda, 256, ldw)) {
+    return SK_ERR_SHAPE;
+  }
   int num_cu = 0;
   if ((st = device_info(&num_cu))) return st;
   int grid = 0;
@@ -1178,6 +1330,21 @@ size_t sk_workspace_bytes(int op, int M, int N, int K, const sk_config* cfg) {
   CallPlan cp;
   if (plan_call(op, M, N, K, cfg, &cp)) return 0;
   return cp.need;
+}
+
+size_t sk_workspace_bytes_preferred(int op, int M, int N, int K) {
+  const size_t least = sk_workspace_bytes(op, M, N, K, nullptr);
+  if (M < 1) return least;
+  size_t want = 0;
+  if (is_handoff_op(op)) {
+    Plan def, pl;
+    if (plan_handoff(op, M, N, K, nullptr, &def) == SK_OK && stream_handoff(op, M, N, K, def, 0, &pl))
+      want = plan_workspace(handoff_base(op), M, N, pl);
+  } else if (is_gemm_family(base_op(op))) {
+    CallPlan cp, alt;
+    if (plan_call(op, M, N, K, nullptr, &cp) == SK_OK && stream_call(op, M, N, K, cp, 0, &alt)) want = alt.need;
+  }
+  return want > least ? want : least;
 }
 
 int sk_gemm_bf16(const sk_bf16* A, int64_t lda, const sk_bf16* W, int64_t ldw, sk_bf16* C, int64_t ldc, int M, int N,

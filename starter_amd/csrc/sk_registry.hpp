@@ -12,6 +12,7 @@
 #include "sk_kernels.hpp"
 #include "sk_wide.hpp"
 #include "sk_wide2.hpp"
+#include "sk_stream.hpp"
 
 namespace sk {
 
@@ -115,6 +116,14 @@ KernelFn wide_for_epi8(int W, int WN, int NT);
 KernelFn wide_for_epi9(int W, int WN, int NT);
 KernelFn wide_for_epi10(int W, int WN, int NT);
 KernelFn wide_for_epi12(int W, int WN, int NT);
+constexpr int stream_key(int KG, int MG, int MT, int NT, int UC) {
+  return (((KG * 10 + MG) * 10 + MT) * 10 + NT) * 1000 + UC;
+}
+KernelFn stream_for_epi0(int KG, int MG, int MT, int NT, int UC);
+KernelFn stream_for_epi1(int KG, int MG, int MT, int NT, int UC);
+KernelFn stream_for_epi3(int KG, int MG, int MT, int NT, int UC);
+KernelFn stream_for_epi11(int KG, int MG, int MT, int NT, int UC);
+KernelFn stream_for_epi12(int KG, int MG, int MT, int NT, int UC);
 KernelFn gemv_for_epi0(int MR, int R, int KU);
 KernelFn gemv_for_epi1(int MR, int R, int KU);
 KernelFn gemv_for_epi2(int MR, int R, int KU);
@@ -181,6 +190,19 @@ inline KernelFn wide_kernel_for(int epi, int W, int WN, int NT) {
     case EPI_SWIGLU_PRE: return wide_for_epi9(W, WN, NT);
     case EPI_ARGMAX_PRE: return wide_for_epi10(W, WN, NT);
     case EPI_PART_RESID: return wide_for_epi12(W, WN, NT);
+  }
+  return nullptr;
+}
+
+// Stream-path instances: KG K groups of MG waves, MT activation tiles per
+// wave, NT slabs of weight rows, UC-column units.
+inline KernelFn stream_kernel_for(int epi, int KG, int MG, int MT, int NT, int UC) {
+  switch (epi) {
+    case EPI_STORE: return stream_for_epi0(KG, MG, MT, NT, UC);
+    case EPI_SWIGLU: return stream_for_epi1(KG, MG, MT, NT, UC);
+    case EPI_PART: return stream_for_epi3(KG, MG, MT, NT, UC);
+    case EPI_STORE_RESID: return stream_for_epi11(KG, MG, MT, NT, UC);
+    case EPI_PART_RESID: return stream_for_epi12(KG, MG, MT, NT, UC);
   }
   return nullptr;
 }

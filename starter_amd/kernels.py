@@ -79,8 +79,11 @@ def _device_guard(t: torch.Tensor) -> None:
 
 def _workspace(op: int, M: int, N: int, K: int, cfg: SkConfig | None, device) -> torch.Tensor | None:
     """Zero-filled once: the library's arrival counters live at its start and
-    every call leaves them at zero again."""
-    n = _lib.workspace_bytes(op, M, N, K, cfg)
+    every call leaves them at zero again.  Without a configuration it is sized
+    for the library's fastest plan, which may split K where the least
+    workspace does not allow it."""
+    n = _lib.workspace_bytes(op, M, N, K, cfg) if cfg is not None or op == SK_OP_ARGMAX else \
+        _lib.workspace_bytes_preferred(op, M, N, K)
     return torch.zeros(n, dtype=torch.uint8, device=device) if n else None
 
 
