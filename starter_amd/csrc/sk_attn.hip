@@ -106,6 +106,93 @@ __global__ void __launch_bounds__(256) qk_norm_rope_kernel(RopeArgs a) {
   }
 }
 
+// The same over 16-byte aligned rows, for prefill and verify row counts: 16
+// lanes per head, lane j (< 8) holding dims 8j .. 8j+7 and lane j + 8 dims
+// 64 + 8j .. +7, so every access is 16 bytes per lane and a rotation pair
+// sits in lanes j and j ^ 8 of one 16-lane row (a DPP row rotation by 8).  The
+// sum of squares is added in rope_head's order (a leaf per pair, a tree over
+// 16 leaves, then the four 16-leaf sums in order; squares of bf16 are exact),
+// so both kernels give the same bits.  A workgroup takes 16 heads of one row,
+// value heads (copied) after the key heads.  Bound by memory: 16 x 1024 rows
+// of 32 + 2 x 8 heads (402 MB) 90-96 us, where one element per lane took
+// 177-182 us.
+__device__ __forceinline__ u32x4 row_swap8(u32x4 v) {
+  u32x4 r;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) r[q] = (uint32_t)__builtin_amdgcn_mov_dpp((int)v[q], 0x128, 0xF, 0xF, false);
+  return r;
+}
+__device__ __forceinline__ float row_lane(float v, int sel) {   // lane 2 * sel of the 16-lane row
+  const int i = __float_as_int(v);
+  switch (sel) {
+    case 0: return __int_as_float(__builtin_amdgcn_mov_dpp(i, 0x150, 0xF, 0xF, false));
+    case 1: return __int_as_float(__builtin_amdgcn_mov_dpp(i, 0x152, 0xF, 0xF, false));
+    case 2: return __int_as_float(__builtin_amdgcn_mov_dpp(i, 0x154, 0xF, 0xF, false));
+    default: return __int_as_float(__builtin_amdgcn_mov_dpp(i, 0x156, 0xF, 0xF, false));
+  }
+}
+__device__ __forceinline__ float bf_at(const u32x4& v, int e) {
+  return bf2f((e & 1) ? v[e >> 1] >> 16 : v[e >> 1] & 0xFFFFu);
+}
+
+__global__ void __launch_bounds__(256) qk_norm_rope_vec_kernel(RopeArgs a) {
+  const int row = blockIdx.x;                       // (b, t)
+  const int head = blockIdx.y * 16 + (threadIdx.x >> 4);
+  const int j = threadIdx.x & 15;                   // lane of the head: dims 8j .. 8j + 7
+  if (head >= a.HQ + 2 * a.HKV) return;             // uniform over the head's 16 lanes
+  const int b = row / a.T, t = row - (row / a.T) * a.T;
+  const int p0 = a.pos[b];
+  const int slot = p0 + t;
+  const int angle = a.depth ? p0 + a.depth[t] : slot;
+  if (angle < 0 || angle >= a.rope_rows) return;
+  const bool is_q = head < a.HQ, is_v = head >= a.HQ + a.HKV;
+  if (!is_q && (slot < 0 || slot >= a.cap)) return;
+  const u32x4 x = ld16_stream(a.qkv + (int64_t)row * a.ld_qkv + (int64_t)head * HEAD_D + 8 * j);
+  if (is_v) {
+    const int kh = head - a.HQ - a.HKV;
+    *reinterpret_cast<u32x4*>(a.v_cache + ((int64_t)(b * a.HKV + kh) * a.cap + slot) * HEAD_D + 8 * j) = x;
+    return;
+  }
+  const u32x4 w = ld16((is_q ? a.qw : a.kw) + 8 * j);
+  const u32x4 c = ld16(a.cos + (int64_t)angle * HEAD_D + 8 * j);
+  const u32x4 s = ld16(a.sin + (int64_t)angle * HEAD_D + 8 * j);
+  const u32x4 xo = row_swap8(x);
+  float leaf[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float p = bf_at(x, e), q = bf_at(xo, e);
+    leaf[e] = p * p + q * q;
+  }
+  const float h = ((leaf[0] + leaf[1]) + (leaf[2] + leaf[3])) + ((leaf[4] + leaf[5]) + (leaf[6] + leaf[7]));
+  const float r = dpp_add(h, 0);                    // the 16-leaf sum, with the neighbour's eight
+  const float ss = ((row_lane(r, 0) + row_lane(r, 1)) + row_lane(r, 2)) + row_lane(r, 3);
+  const float rstd = 1.0f / sqrtf(ss / (float)HEAD_D + a.eps);
+  u32x4 y;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    y[q] = (uint32_t)f2bf(bf_at(w, 2 * q) * round_bf(bf_at(x, 2 * q) * rstd)) |
+           ((uint32_t)f2bf(bf_at(w, 2 * q + 1) * round_bf(bf_at(x, 2 * q + 1) * rstd)) << 16);
+  const u32x4 yo = row_swap8(y);
+  const bool lo = j < 8;
+  u32x4 o;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    uint16_t v[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const float mine = bf_at(y, 2 * q + e), other = bf_at(yo, 2 * q + e), sn = bf_at(s, 2 * q + e);
+      v[e] = f2bf(round_bf(mine * bf_at(c, 2 * q + e)) + round_bf((lo ? -other : other) * sn));
+    }
+    o[q] = (uint32_t)v[0] | ((uint32_t)v[1] << 16);
+  }
+  if (is_q) {
+    *reinterpret_cast<u32x4*>(a.q_out + ((int64_t)(b * a.HQ + head) * a.T + t) * HEAD_D + 8 * j) = o;
+  } else {
+    const int kh = head - a.HQ;
+    *reinterpret_cast<u32x4*>(a.k_cache + ((int64_t)(b * a.HKV + kh) * a.cap + slot) * HEAD_D + 8 * j) = o;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Split-K GQA flash-decoding (attention.py:23-149 numerics: scores and
 // softmax statistics in fp32, probabilities rounded to bf16 before the PV
@@ -655,6 +742,11 @@ int sk_qk_norm_rope_cache_bf16(const sk_bf16* qkv, int64_t ld_qkv, const sk_bf16
   a.HKV = HKV;
   a.cap = cap;
   a.eps = eps;
+  if (aligned16(qkv) && (ld_qkv & 7) == 0 && aligned16(q_norm_w) && aligned16(k_norm_w) && aligned16(cos) &&
+      aligned16(sin) && aligned16(q_out) && aligned16(k_cache) && aligned16(v_cache)) {
+    sk::qk_norm_rope_vec_kernel<<<dim3((unsigned)(B * T), (unsigned)cdiv(HQ + 2 * HKV, 16)), dim3(256), 0, stream>>>(a);
+    return attn_launch_status();
+  }
   const unsigned groups = (unsigned)cdiv(HQ + HKV, 4);
   sk::qk_norm_rope_kernel<<<dim3((unsigned)(B * T), groups), dim3(256), 0, stream>>>(a);
   return attn_launch_status();
