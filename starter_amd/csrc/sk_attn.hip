@@ -8,24 +8,15 @@
 #include "starter_amd.h"
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <math.h>
 #include <string.h>
 
-#include "sk_kernels.hpp"
+#include "sk_stream.hpp"
 
 namespace sk {
 
 constexpr int HEAD_D = 128;   // head width of Qwen3 (the only one compiled)
-
-// K/V blocks a wave keeps in flight beyond the one it processes (1 or 2).
-// One: with two the first round of requests of the whole grid (24 MB at
-// B = 16, position 1088) was served in no particular order and the last waves
-// started late (B = 16 with two key splits: 17.6 us with two blocks ahead,
-// 16.9 with one; pure streaming reads of the same 71 MB by 128 workgroups of
-// 512 threads: 14.6 us with 8 loads per thread in flight, 19.1 with 16).
-#ifndef SK_ATTN_AHEAD
-#define SK_ATTN_AHEAD 1
-#endif
 
 // ---------------------------------------------------------------------------
 // q/k RMSNorm + RoPE + cache write (rope.py:94-188 cast placement):
@@ -198,17 +189,17 @@ __global__ void __launch_bounds__(256) qk_norm_rope_vec_kernel(RopeArgs a) {
 // softmax statistics in fp32, probabilities rounded to bf16 before the PV
 // product, fp32 accumulation, one normalisation at the end).
 //
-// Workgroup (b, kv head, split s): ATTN_WAVES waves stream keys
-// [s*split_len, ...) clipped to the row's valid length pos[b] + t + 1, 16 keys
-// per wave and block.  The scores of the KV head's query rows (QR = G*R of
+// Workgroup (kv head, key range of a sequence, row block): ATTN_WAVES waves
+// stream the range's keys, clipped to the row's valid length pos[b] + t + 1, 16
+// keys per wave and block.  The scores of the KV head's query rows (QR = G*R of
 // them, the columns of a 16-wide MFMA) come from v_mfma_f32_16x16x32_bf16 with
 // the key rows as the A operand; each lane runs the online softmax of its own
 // score column (4 keys of one row per block, the row max shared by the row's
 // 4 lanes through permlane row swaps), and P.V runs on
 // v_mfma_f32_16x16x16_bf16 with the probabilities as they sit in the score
 // layout.  The waves' (m, l, acc) are merged in LDS in wave order.
-// With several splits, the partial (m, l, acc) goes to the workspace and the
-// last workgroup of the (b, kv head) to arrive merges the splits in split
+// With several ranges, the partial (m, l, acc) goes to the workspace and the
+// last workgroup of the (sequence, kv head) to arrive merges the ranges in
 // order (no second kernel).
 // ---------------------------------------------------------------------------
 struct AttnArgs {
@@ -218,10 +209,11 @@ struct AttnArgs {
   const int32_t* pos;       // [B]: position of query row 0
   const int64_t* tree;      // [R] ancestor bit masks, or nullptr for the chain (causal) mask
   uint16_t* out;            // [B, R, HQ, D]
-  float* part_o;            // [B*HKV, NRB, S, QR, D]
-  float* part_ml;           // [B*HKV, NRB, S, QR, 2]
+  float* part_o;            // [B*HKV, S, NRB, QR, D]
+  float* part_ml;           // [B*HKV, S, NRB, QR, 2]
   unsigned* tickets;        // [B*HKV, NRB]
-  int HQ, HKV, R, G, cap, S, split_len, NRB;
+  int B, HQ, HKV, R, G, cap, S, NRB;
+  int cover;                // keys the plan covers (the splits of the planned length)
   float scale;
   // ROPE instances: q rows and the new K/V rows come from the projection
   // buffer (rows (b, t)) through the per-head norm + rotary step.
@@ -255,41 +247,154 @@ __device__ __forceinline__ float rows4_sum(float x) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// VEC floats per lane, device-coherent (sc1), at byte off of descriptor r.
+template <int VEC>
+__device__ __forceinline__ void store_agent_vec(__amdgpu_buffer_rsrc_t r, int off, const float* v) {
+  if constexpr (VEC == 4) {
+    __builtin_amdgcn_raw_buffer_store_b128(
+        u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])}, r, off, 0, 16);
+  } else if constexpr (VEC == 2) {
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(v[0]), __float_as_uint(v[1])}, r, off, 0, 16);
+  } else {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[0]), r, off, 0, 16);
+  }
+}
+template <int VEC>
+__device__ __forceinline__ void load_agent_vec(__amdgpu_buffer_rsrc_t r, int off, float* v) {
+  if constexpr (VEC == 4) {
+    const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 16);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = __uint_as_float(x[e]);
+  } else if constexpr (VEC == 2) {
+    const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 16);
+    v[0] = __uint_as_float(x[0]);
+    v[1] = __uint_as_float(x[1]);
+  } else {
+    v[0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 16));
+  }
+}
+
+// Key ranges.  The host knows only the planned length, so the S ranges of a
+// sequence are cut here, from its own length, in grains of KEY_GRAIN keys:
+// ranges of the planned length left most workgroups of a shorter sequence
+// without keys (one sequence, 2000 of 4096 planned keys: half of them, 14.2 us
+// against 9.9; 4 of 4000 of 8192: 19.8 against 14.4).  A sequence of at most
+// WHOLE_GRAINS keeps one range: another block of 16 keys per wave costs about
+// 0.9 us, publishing and merging ranges 2-3 us (one query row, 300 keys: 7.1 us
+// in one range, 7.3 in three; 16 sequences of 300: 8.7 and 9.9; at 500 keys
+// 9.2 in one or two, 8.1 in four).
+constexpr int KEY_GRAIN = 64, WHOLE_GRAINS = 6;
+struct KeyRange {
+  int pos, len;        // the sequence's position and keys
+  int count, grains;   // its ranges, grains per range (the last may be shorter)
+};
+__device__ __forceinline__ KeyRange key_range(const AttnArgs& a, int b) {
+  KeyRange k;
+  k.pos = a.pos[b];
+  k.len = max(min(min(k.pos + a.R, a.cap), a.cover), 0);
+  const int total = max((k.len + KEY_GRAIN - 1) / KEY_GRAIN, 1);
+  k.grains = total <= WHOLE_GRAINS ? total : max((total + a.S - 1) / a.S, 2);
+  k.count = (total + k.grains - 1) / k.grains;
+  return k;
+}
+
+// A wave's LDS slot: one block of 16 keys (K rows, then V rows); after the
+// keys the space holds the waves' partial accumulators.
+constexpr int KV_SLOT = 2 * 16 * 2 * HEAD_D;
+constexpr int ACC_LD = HEAD_D + 8;   // (the lanes of one f32x4 store hold 16 different rows, and 128-float rows
+                                     // put all of them on the same banks)
+constexpr int attn_lds(int QR, int waves) {
+  const int ring = waves * KV_SLOT, acc = waves * QR * ACC_LD * 4;
+  return ring > acc ? ring : acc;
+}
+
 template <int QR, int ATTN_WAVES, bool TREE, bool ROPE = false>
-__global__ void __launch_bounds__(64 * ATTN_WAVES) decode_attn_kernel(AttnArgs a) {
+__global__ void __launch_bounds__(64 * ATTN_WAVES, 4) decode_attn_kernel(AttnArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) char dyn[];
   __shared__ float s_m[ATTN_WAVES][QR], s_l[ATTN_WAVES][QR];
-  // (rows padded by 8 floats: the lanes of one f32x4 store hold 16 different
-  // rows, and 128-float rows put all of them on the same banks)
-  __shared__ __attribute__((aligned(16))) float s_acc[ATTN_WAVES][QR][HEAD_D + 8];
+  float* const s_acc = reinterpret_cast<float*>(dyn);   // [wave][row][ACC_LD]
   __shared__ int s_last;
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int dg = lane & 15, kr = lane >> 4;
-  // Workgroup (b, kv head, row block, split): query rows rbk*QR .. +QR-1 of
-  // the KV head's G*R rows (row = t*G + g), keys of split s.
-  // With rb_xcd, launch position 8i + x runs row block i mod NRB of the
-  // (b, kv head, split) unit 8(i / NRB) + x: workgroups are dealt to the 8
-  // XCDs round-robin, so the row blocks of one unit run side by side on one
-  // XCD and the later ones read the keys from its L2.
-  const int S = a.S;
-  int bq, s;
+  // Workgroup (key range, sequence, KV head, row block): query rows rbk*QR ..
+  // +QR-1 of the KV head's G*R rows (row = t*G + g).  The range is the slowest
+  // index: ranges that a short sequence does not need leave every XCD alike.
+  // With rb_xcd, launch position 8i + x runs row block i mod NRB of the (range,
+  // sequence, KV head) unit 8(i / NRB) + x: workgroups are dealt to the 8 XCDs
+  // round-robin, so the row blocks of one unit run side by side on one XCD and
+  // the later ones read the keys from its L2.
+  int unit, rbk;
   if (a.rb_xcd) {
     const int i = blockIdx.x >> 3, x = blockIdx.x & 7;
-    const int unit = 8 * (i / a.NRB) + x;
-    s = unit % S;
-    bq = (unit / S) * a.NRB + i % a.NRB;
+    unit = 8 * (i / a.NRB) + x;
+    rbk = i % a.NRB;
   } else {
-    bq = blockIdx.x / S;
-    s = blockIdx.x - (blockIdx.x / S) * S;
+    unit = blockIdx.x / a.NRB;
+    rbk = blockIdx.x - unit * a.NRB;
   }
-  const int bk = bq / a.NRB, rbk = bq - (bq / a.NRB) * a.NRB;
-  const int b = bk / a.HKV, kh = bk - (bk / a.HKV) * a.HKV;
+  const int sb = unit / a.HKV, kh = unit - sb * a.HKV;
+  const int split = sb / a.B, b = sb - split * a.B, bk = b * a.HKV + kh;
+  const KeyRange rng = key_range(a, b);
+  if (split >= rng.count) return;   // uniform: nothing left for this workgroup
   const int rows = a.G * a.R;
-  const int pos = a.pos[b];
-  const int start = s * a.split_len;
-  // keys this workgroup may touch: below the longest row's length and the cache
-  const int end = min(min(start + a.split_len, pos + a.R), a.cap);
+  const int pos = rng.pos;
+  const int start = split * rng.grains * KEY_GRAIN;
+  const int range_end = start + rng.grains * KEY_GRAIN;
+  const bool last_range = split == rng.count - 1;
+  // keys this workgroup may touch: below the longest row's length, the cache
+  // and the planned length
+  const int end = min(range_end, rng.len);
+
+  // Wave w processes the 16-key blocks start + 16 (w + ATTN_WAVES i).  A
+  // block's K and V rows (4 KB each) are loaded straight into the wave's own
+  // LDS slot, four whole 256-byte rows per load, and read back in the layouts
+  // of the two products.  Each half of the slot is loaded again as soon as its
+  // fragments are in registers, so four to eight loads of a wave are always in
+  // flight, and nothing is staged in registers: 119 of them at most, two
+  // workgroups per CU (blocks staged in registers took 180 and one: 64
+  // sequences of up to 200 keys 13.7 us, now 11.5; 5 x 8 tree rows 28.3 us,
+  // now 17.2).  Long contexts are bound by memory (2 x 32000 keys: 42 us, 5.8
+  // TB/s at the mean of both lengths), short ones by the chain of round trips
+  // position, projection row, keys, merge.
+  //  * Scores: S^T[key][row] = K[16 keys, 128] . Q^T by four MFMAs with K as
+  //    the A operand (lane l: key l%16, dims 32s + 8*(l/16)).  Chunk c (16
+  //    bytes) of key r lies at position c ^ r of its row, so the 16 keys of a
+  //    fragment read fall on 16 bank groups.  Lane l then holds keys
+  //    4*(l/16) + i (i < 4) of query row l%16.
+  //  * P.V: lane l reads dims 8*(l%16) .. +7 of keys 4*(l/16) + j, the keys of
+  //    its scores.
+  const uint32_t slot_off =
+      (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)dyn) + wave * KV_SLOT;
+  const char* const slot = dyn + wave * KV_SLOT;
+  const int64_t kv_row0 = (int64_t)bk * a.cap;
+  const int wk0 = start + 16 * wave;
+  const int nblk = wk0 < end ? (end - 1 - wk0) / (16 * ATTN_WAVES) + 1 : 0;   // blocks of this wave (uniform)
+  const int kx16 = 16 * (dg ^ kr);   // chunk dg ^ r of row r = kr + 4 j lies at kx16 ^ 64 j
+  // Keys past `end` in the wave's last block load its last valid row again and
+  // are masked.  K and V rows are read once per launch: non-temporal.
+  auto issue = [&](int i, auto what) {
+    constexpr bool V = decltype(what)::value;
+    const int n0 = wk0 + 16 * ATTN_WAVES * i;
+    const int lim = end - 1 - n0;   // >= 0
+    const i32x4 rows16 = buf_of((V ? a.v : a.k) + (kv_row0 + n0) * HEAD_D, 16 * 2 * HEAD_D);
+    int kr256 = 2 * HEAD_D * kr;   // (the offsets are formed again for each block: eight of them kept would spill)
+    asm volatile("" : "+v"(kr256));
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      load_lds16<true>(slot_off + (V ? 4096 : 0) + 1024 * j,
+                       min(kr256 | (1024 * j), lim * (2 * HEAD_D)) | (V ? 16 * dg : kx16 ^ (64 * j)), rows16, 0);
+  };
+  const std::false_type keys{};
+  const std::true_type values{};
+  // The first block is on its way while the query rows are formed, unless it
+  // holds rows that this launch writes (the caches below pos are not written).
+  const bool early = nblk > 0 && wk0 + 16 <= min(end, pos);   // (uniform)
+  if (early) {
+    issue(0, keys);
+    issue(0, values);
+  }
 
   // Query rows r = t*G + g (head kh*G + g, query row t) as the B operand of
   // v_mfma_f32_16x16x32_bf16: lane l supplies row l%16, dims 32s + 8*(l/16)
@@ -315,7 +420,7 @@ __global__ void __launch_bounds__(64 * ATTN_WAVES) decode_attn_kernel(AttnArgs a
       s_q[r][lane + 64] = o2;
     }
     // The new K/V rows of this (b, kv head) are written by every workgroup
-    // whose key range holds their slot (the last split also takes slots past
+    // whose key range holds their slot (the last range also takes slots past
     // the planned length), before any of its K/V loads: the stores are
     // complete (vmcnt 0) before the barrier.  Only those workgroups read
     // these slots, and each reads them after its own stores; several row
@@ -325,7 +430,7 @@ __global__ void __launch_bounds__(64 * ATTN_WAVES) decode_attn_kernel(AttnArgs a
     constexpr int KV_WAVE0 = QR % ATTN_WAVES;
     for (int t = (wave - KV_WAVE0 + ATTN_WAVES) % ATTN_WAVES; t < T; t += ATTN_WAVES) {   // wave-uniform
       const int slot = pos + t, rot = rot_of(t);
-      const bool mine = slot >= start && (slot < start + a.split_len || s == S - 1);
+      const bool mine = slot >= start && (slot < range_end || last_range);
       if (mine && slot < a.cap && rot >= 0 && rot < a.rope_rows) {
         const uint16_t* row = a.qkv + (int64_t)(b * T + t) * a.ld_qkv;
         uint16_t o1, o2;
@@ -368,71 +473,29 @@ __global__ void __launch_bounds__(64 * ATTN_WAVES) decode_attn_kernel(AttnArgs a
   const bool my_real = r16 < QR && my_gr < rows;
   const int my_t = my_gr / a.G;
   const int row_lim = my_real ? pos + my_t : -1;   // last visible key of the row (chain)
-  long long row_tree = 0ll;
-  if constexpr (TREE) row_tree = my_real ? (long long)a.tree[min(my_t, a.R - 1)] : 0ll;
+  // (ancestor masks wait in LDS for the few masked blocks; every wave stores the
+  // same values and reads them back itself, in order)
+  __shared__ long long s_tree[TREE ? QR : 1];
+  if constexpr (TREE) {
+    if (r16 < QR) s_tree[r16] = my_real ? (long long)a.tree[min(my_t, a.R - 1)] : 0ll;
+  }
 
   float m = -INFINITY, l = 0.f;
   f32x4 acc[8];
 #pragma unroll
   for (int c = 0; c < 8; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // Wave w processes keys n0 + 16w .. n0 + 16w + 15 of each block of
-  // 16 * ATTN_WAVES keys.  K and V are loaded row-contiguously (one load = 4
-  // whole 256-byte rows per wave): load j of lane l holds dims 8*(l%16) .. +7
-  // of key 4j + l/16 for K and of key 4*(l/16) + j for V.
-  //  * Scores: S^T[key][row] = K[16 keys, 128] . Q^T by four MFMAs with K as
-  //    the A operand (lane l: key l%16, dims 32s + 8*(l/16)); the wave's K rows
-  //    pass through its own LDS tile (rows padded to 288 bytes, so neither the
-  //    row writes nor the column reads conflict) into that layout.  Lane l then
-  //    holds keys 4*(l/16) + i (i < 4) of query row l%16.
-  //  * P.V: lane l's V loads hold keys 4*(l/16) + j, the keys of its scores.
-  // The next blocks' rows are loaded while the current one is processed
-  // (keys past `end` reload the last valid row and are masked).
-  constexpr int KPITCH = 2 * HEAD_D + kRowPad;
-  __shared__ __attribute__((aligned(16))) char s_k[ATTN_WAVES][16 * KPITCH];
-  char* const ktile = s_k[wave];
-  const int64_t kv_row0 = (int64_t)bk * a.cap;
-  const int step = 16 * ATTN_WAVES;
-  // K and V rows are read once per launch: non-temporal loads keep them from
-  // displacing other lines in L2 (17.6 vs 19.1 us at B = 16, position 1088).
-  auto load_block = [&](int n0, u32x4* kf, u32x4* vv) {
-    const int base = n0 + 16 * wave;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int kk = max(min(base + 4 * j + kr, end - 1), 0);
-      kf[j] = ld16_stream(a.k + (kv_row0 + kk) * HEAD_D + 8 * dg);
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int kv = max(min(base + 4 * kr + j, end - 1), 0);
-      vv[j] = ld16_stream(a.v + (kv_row0 + kv) * HEAD_D + 8 * dg);
-    }
-  };
-  // Two blocks in flight beyond the one being processed.  Three buffers with
-  // fixed roles rotate through a three-block loop body with a single exit,
-  // so no buffer is ever copied (a loop-carried copy makes the compiler wait
-  // for the prefetched loads at the end of every iteration).  Blocks past
-  // `end` in the last iteration are fully masked; their loads read the last
-  // valid row (one cached line).
   // MASKED: the block may hold keys a row must not see; blocks wholly below
   // min(end, pos) need no masks (every real row sees every key below pos, and
   // padding rows are never written out).
-  auto process = [&](int n0, const u32x4* kf, const u32x4* vv, auto masked) {
+  float p[4];
+  auto softmax = [&](int n0, const f32x4& sacc, auto masked) {
     constexpr bool MASKED = decltype(masked)::value;
-    // K rows into the wave's tile and back in the A-operand layout (LDS
-    // operations of one wave execute in order; the compiler keeps these
-    // accesses in program order since their addresses may alias).
-#pragma unroll
-    for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4*>(ktile + (4 * j + kr) * KPITCH + 16 * dg) = kf[j];
-    f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int st = 0; st < HEAD_D / 32; ++st) {
-      const u32x4 ka = *reinterpret_cast<const u32x4*>(ktile + r16 * KPITCH + 64 * st + 16 * kr);
-      sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ka), qb[st], sacc, 0, 0, 0);
-    }
-    const int key0 = n0 + 16 * wave + 4 * kr;   // keys key0 .. key0+3 of this lane's row
+    const int key0 = n0 + 4 * kr;   // keys key0 .. key0+3 of this lane's row
     float sc[4];
     float mx = m;
+    long long row_tree = 0ll;
+    if constexpr (MASKED && TREE) row_tree = s_tree[min(r16, QR - 1)];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float dot = sacc[j] * a.scale;
@@ -453,7 +516,6 @@ __global__ void __launch_bounds__(64 * ATTN_WAVES) decode_attn_kernel(AttnArgs a
     }
     mx = rows4_max(mx);
     const float msafe = mx == -INFINITY ? 0.f : mx;
-    float p[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) p[j] = __expf(sc[j] - msafe);
     // Rescale only when some row's max moved (alpha == 1 elsewhere, so the
@@ -466,6 +528,35 @@ __global__ void __launch_bounds__(64 * ATTN_WAVES) decode_attn_kernel(AttnArgs a
     }
     l += (p[0] + p[1]) + (p[2] + p[3]);
     m = mx;
+  };
+  const int unmasked_end = min(end, pos);   // keys below it need no masks
+  if (nblk > 0 && !early) {
+    issue(0, keys);
+    issue(0, values);
+  }
+  for (int i = 0; i < nblk; ++i) {
+    const bool more = i + 1 < nblk;
+    const int n0 = wk0 + 16 * ATTN_WAVES * i;
+    wait_loads<4>();   // the keys; the values may be in flight
+    bf16x8 kf[HEAD_D / 32];
+#pragma unroll
+    for (int st = 0; st < HEAD_D / 32; ++st)
+      kf[st] = *reinterpret_cast<const bf16x8*>(slot + 2 * HEAD_D * r16 + 16 * ((4 * st + kr) ^ r16));
+    wait_lds();
+    if (more) issue(i + 1, keys);   // (the keys' half of the slot is in registers)
+    f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int st = 0; st < HEAD_D / 32; ++st)
+      sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[st], qb[st], sacc, 0, 0, 0);
+    if (n0 + 16 <= unmasked_end) softmax(n0, sacc, std::false_type{});   // (uniform)
+    else softmax(n0, sacc, std::true_type{});
+    if (more) wait_loads<4>();   // the values
+    else wait_loads<0>();
+    u32x4 vv[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) vv[j] = *reinterpret_cast<const u32x4*>(slot + 4096 + 2 * HEAD_D * (4 * kr + j) + 16 * dg);
+    wait_lds();
+    if (more) issue(i + 1, values);
     // P.V on MFMA: O^T[dims][rows] += V^T[dims][16 keys] . P^T[16 keys][rows].
     // B = the probabilities as they sit (lane l: row l%16, keys 4*(l/16)+j),
     // rounded to bf16 (RNE) as the reference's tl.dot does; A for dim offset
@@ -480,55 +571,8 @@ __global__ void __launch_bounds__(64 * ATTN_WAVES) decode_attn_kernel(AttnArgs a
         const u32x2 vt = {__builtin_amdgcn_perm(vv[1][c4], vv[0][c4], sel), __builtin_amdgcn_perm(vv[3][c4], vv[2][c4], sel)};
         acc[2 * c4 + h] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, vt), pb, acc[2 * c4 + h], 0, 0, 0);
       }
-  };
-  u32x4 kA[4], vA[4], kB[4], vB[4], kC[4], vC[4];   // the 4 K and 4 V loads of a block
-  const int unmasked_end = min(end, pos);   // keys below it need no masks
-  // Per wave (uniform): its 16 keys of block nb are nb + 16*wave .. +15.  A
-  // wave whose keys all lie at or past `end` skips the block (every score
-  // would be masked: p = 0, m and l unchanged, so skipping is exact); one
-  // whose keys all lie below `unmasked_end` takes the body without masks.
-  auto run = [&](int nb, const u32x4* kf, const u32x4* vv) {
-    const int wk = nb + 16 * wave;
-    if (wk >= end) return;
-    if (wk + 16 <= unmasked_end) process(nb, kf, vv, std::false_type{});
-    else process(nb, kf, vv, std::true_type{});
-  };
-#if SK_ATTN_AHEAD == 1
-  // One block in flight beyond the one being processed (two buffers).
-  (void)kC;
-  (void)vC;
-  if (start < end) load_block(start, kA, vA);
-  for (int n0 = start; n0 < end; n0 += 2 * step) {
-    load_block(n0 + step, kB, vB);
-    __builtin_amdgcn_sched_barrier(0);
-    run(n0, kA, vA);
-    __builtin_amdgcn_sched_barrier(0);
-    load_block(n0 + 2 * step, kA, vA);
-    __builtin_amdgcn_sched_barrier(0);
-    run(n0 + step, kB, vB);
-    __builtin_amdgcn_sched_barrier(0);
   }
-#else
-  if (start < end) {
-    load_block(start, kA, vA);
-    load_block(start + step, kB, vB);
-  }
-  // The scheduling fences keep every prefetch ahead of the block it overlaps.
-  for (int n0 = start; n0 < end; n0 += 3 * step) {
-    load_block(n0 + 2 * step, kC, vC);
-    __builtin_amdgcn_sched_barrier(0);
-    run(n0, kA, vA);
-    __builtin_amdgcn_sched_barrier(0);
-    load_block(n0 + 3 * step, kA, vA);
-    __builtin_amdgcn_sched_barrier(0);
-    run(n0 + step, kB, vB);
-    __builtin_amdgcn_sched_barrier(0);
-    load_block(n0 + 4 * step, kB, vB);
-    __builtin_amdgcn_sched_barrier(0);
-    run(n0 + 2 * step, kC, vC);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-#endif
+  __syncthreads();   // the slots give way to the partial accumulators
 
   // Per wave: the row sums of the 4 lanes of each row, then the waves'
   // results merge in LDS in wave order.
@@ -540,7 +584,7 @@ __global__ void __launch_bounds__(64 * ATTN_WAVES) decode_attn_kernel(AttnArgs a
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      float* dst = &s_acc[wave][r16][8 * (4 * kr + k)];
+      float* dst = s_acc + (wave * QR + r16) * ACC_LD + 8 * (4 * kr + k);
       *reinterpret_cast<f32x4*>(dst) = f32x4{acc[0][k], acc[1][k], acc[2][k], acc[3][k]};
       *reinterpret_cast<f32x4*>(dst + 4) = f32x4{acc[4][k], acc[5][k], acc[6][k], acc[7][k]};
     }
@@ -566,73 +610,104 @@ __global__ void __launch_bounds__(64 * ATTN_WAVES) decode_attn_kernel(AttnArgs a
     s_rowL[r] = L;
   }
   __syncthreads();
-  const bool single = (S == 1);
+  const bool single = rng.count == 1;
   const int nreal = min(QR, rows - rbk * QR);   // rows of this block that exist
-  for (int idx = threadIdx.x; idx < nreal * HEAD_D; idx += 64 * ATTN_WAVES) {
-    const int r = idx / HEAD_D, d = idx - (idx / HEAD_D) * HEAD_D;
-    float O = 0.f;
-#pragma unroll
-    for (int wv = 0; wv < ATTN_WAVES; ++wv) O += s_w[wv][r] * s_acc[wv][r][d];
-    const float L = s_rowL[r];
+  // Every thread takes VEC neighbouring outputs of the QR x HEAD_D.
+  constexpr int VEC = QR * HEAD_D / (64 * ATTN_WAVES);
+  static_assert(VEC * 64 * ATTN_WAVES == QR * HEAD_D && (VEC == 1 || VEC == 2 || VEC == 4), "outputs of a thread");
+  const int r = threadIdx.x * VEC / HEAD_D, d = threadIdx.x * VEC % HEAD_D;
+  auto store_out = [&](const float* O, float L) {
     const int gr = rbk * QR + r;
     const int t = gr / a.G, g = gr - (gr / a.G) * a.G;
-    if (single) {
-      a.out[((int64_t)(b * a.R + t) * a.HQ + kh * a.G + g) * HEAD_D + d] = f2bf(L > 0.f ? O / L : 0.f);
+    uint16_t* const o = a.out + ((int64_t)(b * a.R + t) * a.HQ + kh * a.G + g) * HEAD_D + d;
+    uint16_t y[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) y[e] = f2bf(L > 0.f ? O[e] / L : 0.f);
+    if (VEC > 1 && (reinterpret_cast<uintptr_t>(a.out) & (2 * VEC - 1)) == 0) {   // (uniform)
+      uint32_t w[VEC > 1 ? VEC / 2 : 1];
+#pragma unroll
+      for (int e = 0; e < VEC / 2; ++e) w[e] = (uint32_t)y[2 * e] | ((uint32_t)y[2 * e + 1] << 16);
+      __builtin_memcpy(__builtin_assume_aligned(o, 2 * VEC), w, 2 * VEC);
     } else {
-      const int64_t pr = ((int64_t)bq * S + s) * QR + r;
-      store_agent(&a.part_o[pr * HEAD_D + d], O);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) o[e] = y[e];
+    }
+  };
+  const int64_t part0 = ((int64_t)bk * a.S * a.NRB + rbk) * QR;   // partial row of (range 0, row 0)
+  const int64_t stride = (int64_t)a.NRB * QR;                     // partial rows per range
+  const auto part_rows = [&](int64_t pr, int n) {                 // n partial rows from pr
+    return __builtin_amdgcn_make_buffer_rsrc(a.part_o + pr * HEAD_D, 0, n * HEAD_D * 4, 0x00020000);
+  };
+  {
+    float O[VEC] = {};
+#pragma unroll
+    for (int wv = 0; wv < ATTN_WAVES; ++wv) {
+      float v[VEC];
+      __builtin_memcpy(v, __builtin_assume_aligned(&s_acc[(wv * QR + r) * ACC_LD + d], 4 * VEC), 4 * VEC);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) O[e] += s_w[wv][r] * v[e];
+    }
+    if (single) {
+      if (r < nreal) store_out(O, s_rowL[r]);
+      return;
+    }
+    if (r < nreal) {
+      const int64_t pr = part0 + split * stride;
+      store_agent_vec<VEC>(part_rows(pr, QR), 4 * VEC * threadIdx.x, O);
       if (d == 0) {
-        store_agent(&a.part_ml[2 * pr], s_rowM[r]);
-        store_agent(&a.part_ml[2 * pr + 1], L);
+        store_agent(&a.part_ml[2 * (pr + r)], s_rowM[r]);
+        store_agent(&a.part_ml[2 * (pr + r) + 1], s_rowL[r]);
       }
     }
   }
-  if (single) return;
 
-  // Last workgroup of this (b, kv head) merges the splits in split order.
+  // Last workgroup of this (sequence, KV head, row block) merges the ranges.
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  if (threadIdx.x == 0) s_last = take_ticket(&a.tickets[bq], (unsigned)S) ? 1 : 0;
+  if (threadIdx.x == 0) s_last = take_ticket(&a.tickets[bk * a.NRB + rbk], (unsigned)rng.count) ? 1 : 0;
   __syncthreads();
-  if (!s_last) return;
-  // Each output loads its splits' (m, l, o) in batches of MB, all loads of a
-  // batch issued before any arithmetic (one memory round trip per batch, not
-  // one per split); the merge itself runs in split order 0..S-1.
-  constexpr int MB = 4;
-  for (int idx = threadIdx.x; idx < QR * HEAD_D; idx += 64 * ATTN_WAVES) {
-    const int r = idx / HEAD_D, d = idx - (idx / HEAD_D) * HEAD_D;
-    const int gr = rbk * QR + r;
-    const int t = gr / a.G, g = gr - (gr / a.G) * a.G;
-    if (gr >= rows) continue;
-    const int64_t pr0 = (int64_t)bq * S * QR + r;   // split sp: pr0 + sp * QR
-    float M = -INFINITY;
-    for (int s0 = 0; s0 < S; s0 += MB) {
-      float ms[MB];
+  if (!s_last || r >= nreal) return;
+  // A thread folds its outputs of the ranges in order, a batch at a time with
+  // all its loads issued before any arithmetic: the merge is a chain of memory
+  // round trips, one per batch (one row, 32 ranges: two trips instead of the 16
+  // of a pass over the maxima and batches of four).
+  float M = -INFINITY, L = 0.f, O[VEC] = {};
+  const auto fold = [&](int s0, auto batch) {
+    constexpr int MB = decltype(batch)::value;
+    const int n = min(rng.count - s0, MB);
+    const auto src = part_rows(part0 + s0 * stride, (int)((n - 1) * stride) + QR);
+    float ms[MB], ls[MB], os[MB][VEC];
 #pragma unroll
-      for (int k = 0; k < MB; ++k) ms[k] = load_agent(&a.part_ml[2 * (pr0 + (int64_t)min(s0 + k, S - 1) * QR)]);
-#pragma unroll
-      for (int k = 0; k < MB; ++k) M = fmaxf(M, ms[k]);   // repeats of split S-1 change nothing
+    for (int k = 0; k < MB; ++k) {
+      const int s = min(k, n - 1);   // (past the end: the last again, not added)
+      const int64_t pr = part0 + (s0 + s) * stride + r;
+      ms[k] = load_agent(&a.part_ml[2 * pr]);
+      ls[k] = load_agent(&a.part_ml[2 * pr + 1]);
+      load_agent_vec<VEC>(src, (int)(s * stride) * (HEAD_D * 4) + 4 * VEC * (int)threadIdx.x, os[k]);
     }
-    float L = 0.f, O = 0.f;
-    for (int s0 = 0; s0 < S; s0 += MB) {
-      float ms[MB], ls[MB], os[MB];
+    float Mb = M;
 #pragma unroll
-      for (int k = 0; k < MB; ++k) {
-        const int64_t pr = pr0 + (int64_t)min(s0 + k, S - 1) * QR;
-        ms[k] = load_agent(&a.part_ml[2 * pr]);
-        ls[k] = load_agent(&a.part_ml[2 * pr + 1]);
-        os[k] = load_agent(&a.part_o[pr * HEAD_D + d]);
-      }
+    for (int k = 0; k < MB; ++k) Mb = fmaxf(Mb, ms[k]);
+    if (Mb == -INFINITY) return;   // no visible key so far
+    const float keep = __expf(M - Mb);   // 0 before the first visible key
+    L *= keep;
 #pragma unroll
-      for (int k = 0; k < MB; ++k) {
-        if (s0 + k >= S) break;
-        const float w = ms[k] == -INFINITY ? 0.f : __expf(ms[k] - M);
+    for (int e = 0; e < VEC; ++e) O[e] *= keep;
+    M = Mb;
+#pragma unroll
+    for (int k = 0; k < MB; ++k) {
+      if (k < n) {
+        const float w = __expf(ms[k] - M);
         L += w * ls[k];
-        O += w * os[k];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) O[e] += w * os[k][e];
       }
     }
-    a.out[((int64_t)(b * a.R + t) * a.HQ + kh * a.G + g) * HEAD_D + d] = f2bf(L > 0.f ? O / L : 0.f);
-  }
+  };
+  int s0 = 0;
+  for (; rng.count - s0 > 8; s0 += 16) fold(s0, std::integral_constant<int, 16>{});
+  if (s0 < rng.count) fold(s0, std::integral_constant<int, 8>{});
+  store_out(O, L);
 }
 
 }  // namespace sk
@@ -762,6 +837,17 @@ size_t sk_decode_attention_workspace_bytes(int B, int HQ, int HKV, int D, int R,
 
 namespace {
 
+template <int QR, bool TREE, bool ROPE>
+int attn_launch(const sk::AttnArgs& a, unsigned grid, hipStream_t stream) {
+  constexpr int lds = sk::attn_lds(QR, kAttnWaves);
+  const auto fn = &sk::decode_attn_kernel<QR, kAttnWaves, TREE, ROPE>;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, lds) !=
+      hipSuccess)
+    return SK_ERR_LAUNCH;
+  fn<<<dim3(grid), dim3(64 * kAttnWaves), lds, stream>>>(a);
+  return attn_launch_status();
+}
+
 // Fills the plan-dependent fields of a and launches the instance for
 // (QR, tree, rope).
 int attn_run(const AttnPlan& p, sk::AttnArgs& a, int B, int HQ, int HKV, int R, int cap, float scale, void* ws,
@@ -777,31 +863,23 @@ int attn_run(const AttnPlan& p, sk::AttnArgs& a, int B, int HQ, int HKV, int R, 
   a.R = R;
   a.G = HQ / HKV;
   a.cap = cap;
+  a.B = B;
   a.S = p.S;
-  a.split_len = p.split_len;
+  a.cover = (int)std::min<int64_t>((int64_t)p.S * p.split_len, cap);
   a.NRB = p.NRB;
   a.rb_xcd = p.NRB > 1 && (B * HKV * p.S) % 8 == 0;
   a.scale = scale;
-  const dim3 grid((unsigned)(B * HKV * p.NRB * p.S));
-  const dim3 block(64 * kAttnWaves);
-  if (rope && a.tree) {
-    if (p.QR == 4) sk::decode_attn_kernel<4, kAttnWaves, true, true><<<grid, block, 0, stream>>>(a);
-    else if (p.QR == 8) sk::decode_attn_kernel<8, kAttnWaves, true, true><<<grid, block, 0, stream>>>(a);
-    else sk::decode_attn_kernel<16, kAttnWaves, true, true><<<grid, block, 0, stream>>>(a);
-  } else if (rope) {
-    if (p.QR == 4) sk::decode_attn_kernel<4, kAttnWaves, false, true><<<grid, block, 0, stream>>>(a);
-    else if (p.QR == 8) sk::decode_attn_kernel<8, kAttnWaves, false, true><<<grid, block, 0, stream>>>(a);
-    else sk::decode_attn_kernel<16, kAttnWaves, false, true><<<grid, block, 0, stream>>>(a);
-  } else if (a.tree) {
-    if (p.QR == 4) sk::decode_attn_kernel<4, kAttnWaves, true><<<grid, block, 0, stream>>>(a);
-    else if (p.QR == 8) sk::decode_attn_kernel<8, kAttnWaves, true><<<grid, block, 0, stream>>>(a);
-    else sk::decode_attn_kernel<16, kAttnWaves, true><<<grid, block, 0, stream>>>(a);
-  } else {
-    if (p.QR == 4) sk::decode_attn_kernel<4, kAttnWaves, false><<<grid, block, 0, stream>>>(a);
-    else if (p.QR == 8) sk::decode_attn_kernel<8, kAttnWaves, false><<<grid, block, 0, stream>>>(a);
-    else sk::decode_attn_kernel<16, kAttnWaves, false><<<grid, block, 0, stream>>>(a);
-  }
-  return attn_launch_status();
+  const unsigned grid = (unsigned)(B * HKV * p.NRB * p.S);
+  const auto launch = [&](auto tree_c, auto rope_c) {
+    constexpr bool TREE = decltype(tree_c)::value, ROPE = decltype(rope_c)::value;
+    if (p.QR == 4) return attn_launch<4, TREE, ROPE>(a, grid, stream);
+    if (p.QR == 8) return attn_launch<8, TREE, ROPE>(a, grid, stream);
+    return attn_launch<16, TREE, ROPE>(a, grid, stream);
+  };
+  const std::true_type yes{};
+  const std::false_type no{};
+  if (rope) return a.tree ? launch(yes, yes) : launch(no, yes);
+  return a.tree ? launch(yes, no) : launch(no, no);
 }
 
 bool overlaps(const void* a, size_t na, const void* b, size_t nb) {

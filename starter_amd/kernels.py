@@ -506,10 +506,10 @@ def qk_norm_rope_cache(qkv: torch.Tensor, q_norm_w: torch.Tensor, k_norm_w: torc
 
 class DecodeAttention:
     """Workspace-owning wrapper; one instance per (B, HQ, cap) plan
-    (engine/kernels/attention.py:152-202).  Split count and key ranges are
-    fixed at construction from ``maxlen`` (default cap); the valid length of
-    each sequence is read from ``pos`` on the device at every call, so one
-    instance replays inside a graph while the sequences grow.  ``R`` query rows
+    (engine/kernels/attention.py:152-202).  The split count is fixed at
+    construction from ``maxlen`` (default cap); the valid length of each
+    sequence is read from ``pos`` on the device at every call and its key ranges
+    are cut there, so one instance replays inside a graph while the sequences grow.  ``R`` query rows
     per sequence (speculative verify), chain-masked, or with ``tree=True``
     masked by per-row ancestor bit masks passed at call time.
     ``block_n``/``num_warps``/``num_stages`` are accepted for signature
