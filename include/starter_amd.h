@@ -137,6 +137,9 @@ typedef enum sk_path {
  *            columns per tile (up to 80, gate/up up to 40), grid 0 (one
  *            workgroup per tile and split); no fused argmax, gate/up with one
  *            split, of the hand-off ops the producer (rows a multiple of 16).
+ *            With grid > 0 it runs persistent tiles, for plain products and
+ *            the fused argmax: waves 8, ku 2, rows 160, split 1, groups 4;
+ *            up to `grid` workgroups share the 16-row slabs evenly.
  *
  * Rows per launch: at most 64 without row groups; with a configuration that
  * splits them into groups (compiled for groups of up to 32 rows), up to 128

@@ -40,7 +40,7 @@ N_EPI = 5       # EPI_STORE, EPI_SWIGLU, EPI_ARGMAX, EPI_PART, EPI_PART_GU
 NORM_EPIS = (5, 6, 7)   # the first three with the norm prologue (GEMV path only)
 HANDOFF_EPIS = (8, 9, 10, 11, 12)   # residual hand-off consumers and producers (LDS-fed ring path)
 WIDE_HANDOFF_EPIS = (8, 9, 10, 12)   # the same on the two-operand wide path (no bf16-store producer)
-STREAM_EPIS = (0, 1, 3, 11, 12)   # stream path: store, SwiGLU, split-K partials and the residual producers
+STREAM_EPIS = (0, 1, 2, 3, 11, 12)   # stream path: store, SwiGLU, argmax, split-K partials and the residual producers
 
 
 def _units() -> list[tuple[Path, list[str], Path]]:

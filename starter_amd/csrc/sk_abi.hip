@@ -123,6 +123,7 @@ struct Plan {
   size_t stage_elem = 0;        // LDS bytes per staged tile (0: argmax keeps 8*M bytes)
   size_t lds = 0;               // total dynamic LDS (set once the grid is known)
   int uc = 0, mg = 0;           // stream path: columns per unit, waves per K group
+  int slabs_n = 0;              // stream path, persistent tiles: weight rows
   size_t ticket_min = 0;        // least bytes of the workspace's counter area
   bool norm = false;            // the op has the add + RMSNorm prologue
   bool fused = false;           // ... and it runs inside the projection kernel
@@ -172,6 +173,7 @@ sk::KernelFn plan_kernel(const Plan& pl) {
   if (pl.cfg.path == SK_PATH_MFMA) return sk::mfma_kernel_for(pl.epi, pl.tm, pl.tn, pl.tku);
   if (pl.cfg.path == SK_PATH_WIDE)
     return sk::wide_kernel_for(pl.epi, pl.cfg.waves, pl.cfg.groups > 1 ? pl.cfg.groups : 1, pl.tn);
+  if (pl.cfg.path == SK_PATH_STREAM && pl.cfg.grid > 0) return sk::stream_tiles_kernel_for(pl.epi, pl.tm);
   if (pl.cfg.path == SK_PATH_STREAM)
     return sk::stream_kernel_for(pl.epi, pl.cfg.waves / pl.mg, pl.mg, pl.tm, pl.tn, pl.uc);
   if (pl.cfg.path == SK_PATH_MFMA_LDS)
@@ -227,6 +229,7 @@ int plan_shape_impl(int op, int M, int N, int K, const sk_config& c, bool fused,
     if (fused) return SK_ERR_CONFIG;
     if (variant == 2 && op != SK_OP_GEMM) return SK_ERR_CONFIG;
     if (c.path == SK_PATH_STREAM) {
+      if (c.grid != 0) return SK_ERR_CONFIG;
       // producers only, in tiles of whole 16-column groups (the finish writes
       // one partial sum per group)
       if (variant != 2 || (c.rows & 15) != 0) return SK_ERR_CONFIG;
@@ -305,6 +308,20 @@ int plan_shape_impl(int op, int M, int N, int K, const sk_config& c, bool fused,
     pl->tku = sk::kWideChunk;
     partial_rows = 0;
     pl->pre_lds = wn == 4 ? sk::wide2_lds(pl->tn) : sk::wide_weight_lds(pl->tn);
+  } else if (c.path == SK_PATH_STREAM && c.grid > 0) {
+    // Persistent tiles: eight waves in four row groups, 64-column units,
+    // 160-row tiles, `grid` workgroups at most.
+    if (gateup || c.split != 1 || c.waves != 8 || c.groups != sk::kTilesMG || 32 * c.ku != sk::kTilesUC ||
+        c.rows != sk::kTilesRows || c.grid > kMaxGrid || K % sk::kTilesUC != 0)
+      return SK_ERR_CONFIG;
+    units = K / sk::kTilesUC;
+    pl->uc = pl->tku = sk::kTilesUC;
+    pl->mg = c.groups;
+    pl->tm = cdiv(M, 16 * c.groups);
+    pl->tn = sk::kTilesNT * sk::kTilesNG;
+    pl->slabs_n = N;
+    partial_rows = 0;
+    pl->pre_lds = sk::tiles_lds(pl->tm);
   } else if (c.path == SK_PATH_STREAM) {
     // waves = KG * MG, MG = groups; MT and NT follow from the rows.
     const int mg = c.groups > 1 ? c.groups : 1;
@@ -596,8 +613,21 @@ const StreamEntry kStream[] = {
     {SK_OP_RESID_GEMM, 2560, 9728, 65, 128, {5, 4, 4, 32, 3, 0, 4}},    // down 96 rows 24.8 (27.5), 128 27.7 (31.4)
 };
 
+// Persistent tiles (sk_stream.hpp), by size and not by shape: weight rows for
+// at least one whole tile on each of the 256 CUs, and enough activation rows
+// that sharing them across tall tiles pays.  151936 x 2560 weights, us, this
+// plan against the table's: logits at 32 rows 131.4 (130.0), 33 133.7 (137.0),
+// 128 176.7 (203.1); fused argmax at 48 rows 127.4 (123.0), 64 130.8 (144.9),
+// 128 150.7 (191.5).
+const StreamEntry kTilesLogits = {SK_OP_GEMM, 0, 0, 33, kMaxLaunchM, {5, 8, 2, sk::kTilesRows, 1, 256, sk::kTilesMG}};
+const StreamEntry kTilesArgmax = {SK_OP_LM_ARGMAX, 0, 0, 49, kMaxLaunchM, {5, 8, 2, sk::kTilesRows, 1, 256, sk::kTilesMG}};
+
 // The n-th stream entry of op/N/K at M rows, or nullptr.
 const StreamEntry* stream_lookup(int op, int M, int N, int K, int n) {
+  if ((op == SK_OP_GEMM || op == SK_OP_LM_ARGMAX) && N >= 256 * sk::kTilesRows && K % sk::kTilesUC == 0) {
+    const StreamEntry& e = op == SK_OP_GEMM ? kTilesLogits : kTilesArgmax;
+    return n == 0 && e.m_lo <= M && M <= e.m_hi ? &e : nullptr;
+  }
   for (const StreamEntry& e : kStream)
     if (e.op == op && e.N == N && e.K == K && e.m_lo <= M && M <= e.m_hi && n-- == 0) return &e;
   return nullptr;
@@ -776,7 +806,10 @@ int bind_plan(Plan* pl, int num_cu, int* grid) {
   if (threads > fi.max_threads) return SK_ERR_CONFIG;
   pl->fn = fn;
   const int S = pl->cfg.split;
-  if (pl->cfg.path == SK_PATH_STREAM) {   // one workgroup per tile and split
+  if (pl->cfg.path == SK_PATH_STREAM && pl->cfg.grid > 0) {   // persistent: every workgroup a 16-row slab at least
+    const int slabs = cdiv(pl->slabs_n, 16);
+    *grid = slabs < pl->cfg.grid ? slabs : pl->cfg.grid;
+  } else if (pl->cfg.path == SK_PATH_STREAM) {   // one workgroup per tile and split
     *grid = pl->nrb * S;
   } else if (pl->cfg.grid > 0) {
     *grid = pl->cfg.grid;

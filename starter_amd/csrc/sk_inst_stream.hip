@@ -1,4 +1,4 @@
-// Stream-path kernel instances (sk_stream.hpp) for one epilogue (-DSK_EPI=<0, 1, 3, 11, 12>).
+// Stream-path kernel instances (sk_stream.hpp) for one epilogue (-DSK_EPI=<0, 1, 2, 3, 11, 12>).
 #include "sk_registry.hpp"
 
 #ifndef SK_EPI
@@ -10,6 +10,18 @@
 
 namespace sk {
 
+#if SK_EPI == 0 || SK_EPI == 2   // persistent tiles: logits and the fused argmax
+template <int MT, int EPI>
+__global__ void __launch_bounds__(64 * kTilesMG * kTilesNG) stream_tiles_entry(Args p) {
+  stream_tiles_body<MT, EPI>(p);
+}
+
+KernelFn SK_CAT(stream_tiles_for_epi, SK_EPI)(int MT) {
+  return MT == 1 ? &stream_tiles_entry<1, SK_EPI> : MT == 2 ? &stream_tiles_entry<2, SK_EPI> : nullptr;
+}
+#endif
+
+#if SK_EPI != 2
 template <int KG, int MG, int MT, int NT, int UC, int EPI>
 __global__ void __launch_bounds__(64 * KG * MG) stream_entry(Args p) {
   stream_body<KG, MG, MT, NT, UC, EPI>(p);
@@ -31,5 +43,6 @@ KernelFn SK_CAT(stream_for_epi, SK_EPI)(int KG, int MG, int MT, int NT, int UC) 
   }
   return nullptr;
 }
+#endif
 
 }  // namespace sk

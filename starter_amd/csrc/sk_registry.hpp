@@ -124,6 +124,8 @@ KernelFn stream_for_epi1(int KG, int MG, int MT, int NT, int UC);
 KernelFn stream_for_epi3(int KG, int MG, int MT, int NT, int UC);
 KernelFn stream_for_epi11(int KG, int MG, int MT, int NT, int UC);
 KernelFn stream_for_epi12(int KG, int MG, int MT, int NT, int UC);
+KernelFn stream_tiles_for_epi0(int MT);
+KernelFn stream_tiles_for_epi2(int MT);
 KernelFn gemv_for_epi0(int MR, int R, int KU);
 KernelFn gemv_for_epi1(int MR, int R, int KU);
 KernelFn gemv_for_epi2(int MR, int R, int KU);
@@ -203,6 +205,15 @@ inline KernelFn stream_kernel_for(int epi, int KG, int MG, int MT, int NT, int U
     case EPI_PART: return stream_for_epi3(KG, MG, MT, NT, UC);
     case EPI_STORE_RESID: return stream_for_epi11(KG, MG, MT, NT, UC);
     case EPI_PART_RESID: return stream_for_epi12(KG, MG, MT, NT, UC);
+  }
+  return nullptr;
+}
+
+// Persistent tiles of the stream path: MT activation tiles per row group.
+inline KernelFn stream_tiles_kernel_for(int epi, int MT) {
+  switch (epi) {
+    case EPI_STORE: return stream_tiles_for_epi0(MT);
+    case EPI_ARGMAX: return stream_tiles_for_epi2(MT);
   }
   return nullptr;
 }

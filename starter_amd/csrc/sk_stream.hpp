@@ -386,4 +386,257 @@ __device__ __forceinline__ void stream_body(const Args& p) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Persistent tiles: many more weight rows than one tile per CU holds (a
+// vocabulary head).  One workgroup of eight waves per CU walks a contiguous
+// range of the 16-row slabs in tiles of kTilesRows rows; the ring runs on across
+// the tiles, so the next tile's first units are in flight while a tile is
+// finished.  The waves are four row groups of MT activation tiles by two
+// column groups of NT slabs, and share every unit of 64 columns.
+//
+// What bounds it.  Each tile reads the activation rows again (from L2), so the
+// bytes through a CU per weight row fall with the tile's height: 160 rows is
+// the most that leaves a ring four units deep beside 128 activation rows
+// (36 KB a unit).  The slabs are dealt out evenly (they differ by one between
+// workgroups) and start on 16 columns, so a row's four lanes store whole
+// 32-byte pieces straight from the accumulators.
+// Measured over 151936 x 2560 weights (two-operand wide path before): logits
+// at 128 rows 203 -> 177 us, 96 rows 176 -> 169, 64 rows 157 -> 152, 40 rows
+// 142 -> 137; fused argmax 128 rows 191 -> 151 (5.2 TB/s of weights), 96 rows
+// 159 -> 145, 64 rows 145 -> 131.  The logits' 39 MB of stores cost the
+// difference of the two.
+// ---------------------------------------------------------------------------
+constexpr int kTilesMG = 4, kTilesNG = 2, kTilesNT = 5, kTilesUC = 64;
+constexpr int kTilesRows = 16 * kTilesNG * kTilesNT;
+constexpr int tiles_slot(int MT) { return (kTilesMG * MT * 16 + kTilesRows) * 2 * kTilesUC; }
+constexpr int tiles_lds(int MT) { return 4 * tiles_slot(MT); }
+
+template <int MT, int EPI>
+__device__ __forceinline__ void stream_tiles_body(const Args& p) {
+  constexpr int BASE = EpiTraits<EPI>::base;
+  static_assert(BASE == EPI_STORE || BASE == EPI_ARGMAX, "epilogues of the persistent tiles");
+  static_assert(!EpiTraits<EPI>::norm && !EpiTraits<EPI>::pre && !EpiTraits<EPI>::resid, "plain operands");
+  constexpr int MG = kTilesMG, NT = kTilesNT, UC = kTilesUC, W = kTilesMG * kTilesNG, D = 4;
+  constexpr int KS = UC / 32;
+  constexpr int WB = kTilesRows / 8, AB = MG * MT * 2;   // loads (8 rows each) of a unit's weights and activations
+  constexpr int NI = (WB + AB + W - 1) / W;              // loads per wave and unit (the last may repeat one)
+  constexpr int SLOT = tiles_slot(MT);
+  static_assert(SLOT == (WB + AB) * 1024 && tiles_lds(MT) <= kStreamLds - 2048, "ring and argmax bests fit the LDS");
+
+  extern __shared__ __attribute__((aligned(1024))) float lds[];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int mg = wave % MG, ng = wave / MG;
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int M = p.M, N = p.N;
+  const int units = p.K / UC;   // the host guarantees K % UC == 0
+  // this workgroup's slabs [lo, hi) and tiles (the host launches no more
+  // workgroups than slabs)
+  const int slabs = (N + 15) >> 4, wg = blockIdx.x, nwg = gridDim.x;
+  const int each = slabs / nwg, extra = slabs - each * nwg;
+  const int lo = wg * each + min(wg, extra), hi = lo + each + (wg < extra ? 1 : 0);
+  const int n_hi = min(16 * hi, N);
+  const int ntiles = (hi - lo + kTilesRows / 16 - 1) / (kTilesRows / 16);
+  const int total = ntiles * units;
+
+  unsigned long long* const lds_best =
+      reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(lds) + tiles_lds(MT));
+  if constexpr (BASE == EPI_ARGMAX)
+    for (int i = tid; i < M; i += 64 * W) lds_best[i] = 0ull;   // ordered by the first unit's barrier
+
+  const char* const ring = reinterpret_cast<const char*>(lds);
+  const uint32_t ring_off =
+      (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)reinterpret_cast<char*>(lds));
+
+  // Load q of a unit covers rows 8q .. 8q + 7 of the slot: the tile's weight
+  // rows, then the activation rows; wave w issues loads w, w + W, ...  Rows
+  // past a tile's last lie past the descriptor (row strides are at least K),
+  // as does the offset that rows past M get.
+  auto sw = [](int r) { return (r & 15) >> 1; };
+  int off[NI], slot_at[NI];
+#pragma unroll
+  for (int j = 0; j < NI; ++j) {
+    const int q = min(j * W + wave, WB + AB - 1);
+    const bool weight = q < WB;
+    const int r = 8 * (weight ? q : q - WB) + (lane >> 3);
+    const int at = 16 * ((lane & 7) ^ sw(r));
+    off[j] = weight ? r * (int)p.ldw * 2 + at : r < M ? r * (int)p.lda * 2 + at : 0x7FFF0000;
+    slot_at[j] = q * 1024;
+  }
+  const i32x4 buf_a = buf_of(p.A, ((M - 1) * (int)p.lda + p.K) * 2);
+  i32x4 buf_w;
+  auto weights_of = [&](int t) {
+    const int n0 = 16 * lo + kTilesRows * t;
+    const int cols = min(kTilesRows, n_hi - n0);
+    buf_w = buf_of(p.W0 + (int64_t)n0 * p.ldw, ((cols - 1) * (int)p.ldw + p.K) * 2);
+  };
+  auto load1 = [&](int j, int so, uint32_t base) {
+    if (j * W + W <= WB || (j * W < WB && j * W + wave < WB))   // (uniform)
+      load_lds16<true>(base + slot_at[j], off[j], buf_w, so);
+    else
+      load_lds16<false>(base + slot_at[j], off[j], buf_a, so);
+  };
+  int foff[KS];   // chunk g4 + 4u of row r16 of every slab
+#pragma unroll
+  for (int u = 0; u < KS; ++u) foff[u] = (r16 >> 3) * 1024 + 16 * ((r16 & 7) * 8 + ((g4 + 4 * u) ^ sw(r16)));
+
+  f32x4 acc[NT][MT];
+  auto zero_acc = [&]() {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  zero_acc();
+  struct Frags {
+    bf16x8 w[KS][NT], a[KS][MT];
+  };
+  auto read = [&](int slot, Frags& f) {
+    const char* const b = ring + slot * SLOT;
+#pragma unroll
+    for (int u = 0; u < KS; ++u) {
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+        f.w[u][nt] = *reinterpret_cast<const bf16x8*>(b + (ng * NT + nt) * 2048 + foff[u]);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        f.a[u][mt] = *reinterpret_cast<const bf16x8*>(b + WB * 1024 + (mg * MT + mt) * 2048 + foff[u]);
+    }
+  };
+  constexpr int TOT = KS * MT * NT;
+  auto multiply = [&](const Frags& f, auto fill, int so, uint32_t base) {
+#pragma unroll
+    for (int k = 0; k < TOT; ++k) {
+      const int u = k / (MT * NT), mt = (k / NT) % MT, nt = k % NT;
+      if constexpr (decltype(fill)::value) {
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+          if (j * TOT / NI == k) {
+            __builtin_amdgcn_sched_barrier(0);
+            load1(j, so, base);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+      }
+      acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[u][nt], f.a[u][mt], acc[nt][mt], 0, 0, 0);
+    }
+  };
+  // Lane l holds columns 4 * (l / 16) .. + 3 of each slab for row l % 16.
+  // (Counting a tile's stores in the waits of the next units instead of
+  // draining them changed nothing.)
+  const bool vec = ((p.ldc & 3) == 0) && (reinterpret_cast<uintptr_t>(p.C) & 7) == 0;
+  auto finish = [&](int t) {
+    const int n0 = 16 * lo + kTilesRows * t + 16 * NT * ng + 4 * g4;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int m = 16 * (mg * MT + mt) + r16;
+      if constexpr (BASE == EPI_ARGMAX) {
+        uint32_t bo = 0u;
+        int bn = 0;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int n = n0 + 16 * nt + e;
+            const uint32_t o = argmax_ord(f2bf(acc[nt][mt][e]));
+            if (n < n_hi && o > bo) {   // increasing columns: ties keep the lowest
+              bo = o;
+              bn = n;
+            }
+          }
+        unsigned long long key = bo ? argmax_pack(bo, bn) : 0ull;
+#pragma unroll
+        for (int x = 16; x <= 32; x <<= 1) {
+          const unsigned long long o = ((unsigned long long)(uint32_t)__shfl_xor((int)(key >> 32), x) << 32) |
+                                       (uint32_t)__shfl_xor((int)(key & 0xFFFFFFFFu), x);
+          key = o > key ? o : key;
+        }
+        if (g4 == 0 && m < M && key) atomicMax(&lds_best[m], key);
+      } else if (m < M) {
+        uint16_t* const row = p.C + (int64_t)m * p.ldc;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          const int n = n0 + 16 * nt;
+          uint16_t y[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[e] = f2bf(acc[nt][mt][e]);
+          if (vec && n + 4 <= n_hi) {
+            *reinterpret_cast<u32x2*>(row + n) =
+                u32x2{(uint32_t)y[0] | ((uint32_t)y[1] << 16), (uint32_t)y[2] | ((uint32_t)y[3] << 16)};
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (n + e < n_hi) row[n + e] = y[e];
+          }
+        }
+      }
+    }
+  };
+  // The loads run D units ahead: unit lu of tile lt is the next to request.
+  int lt = 0, lu = 0;
+  auto advance_loads = [&]() {
+    if (++lu == units) {
+      lu = 0;
+      if (++lt < ntiles) weights_of(lt);
+    }
+  };
+  int ct = 0, cu = 0;   // the unit being multiplied
+  // As in stream_body: unit i's fragments are in cur, its slot (sc) is free
+  // past the barrier; unit i + 1 is in slot sn once every wave's loads of it
+  // have landed.  (The stores of a finished tile count as outstanding too:
+  // they only make the wait stricter.)
+  auto step = [&](int i, const Frags& cur, Frags& next, int sc, int sn) {
+    if (i + 1 < total) {
+      if (i + D <= total) wait_loads<(D - 2) * NI>();
+      else wait_loads<0>();
+      wait_lds();
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      read(sn, next);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (i + D < total) {
+      multiply(cur, std::true_type{}, 2 * UC * lu, ring_off + sc * SLOT);
+      advance_loads();
+    } else {
+      multiply(cur, std::false_type{}, 0, 0u);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (++cu == units) {
+      finish(ct);
+      __builtin_amdgcn_sched_barrier(0);
+      zero_acc();
+      cu = 0;
+      ++ct;
+    }
+  };
+  weights_of(0);
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (d < total) {
+#pragma unroll
+      for (int j = 0; j < NI; ++j) load1(j, 2 * UC * lu, ring_off + d * SLOT);
+      advance_loads();
+    }
+  if (total >= D) wait_loads<(D - 1) * NI>();
+  else wait_loads<0>();
+  wait_lds();   // (the argmax bests)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  Frags f0, f1;
+  read(0, f0);
+  int i = 0, sc = 0;
+  for (; i + 1 < total; i += 2) {
+    step(i, f0, f1, sc, (sc + 1) & (D - 1));
+    step(i + 1, f1, f0, (sc + 1) & (D - 1), (sc + 2) & (D - 1));
+    sc = (sc + 2) & (D - 1);
+  }
+  if (i < total) step(i, f0, f1, sc, (sc + 1) & (D - 1));
+
+  if constexpr (BASE == EPI_ARGMAX) {
+    __syncthreads();
+    argmax_fixup(p, lds_best, reinterpret_cast<int*>(lds_best + M));
+  }
+}
+
 }  // namespace sk

@@ -105,6 +105,74 @@ def test_stream_residual_producer(N, Kd, cfg, M):
     assert torch.allclose(sq.double(), padded.pow(2).view(M, -1, 16).sum(-1), rtol=8 * 2.0 ** -24, atol=0)
 
 
+# Persistent tiles: workgroups with unequal slabs, a ragged last slab, last
+# tiles of one slab, fewer units than the ring is deep, odd unit counts (the
+# fragment registers swap roles from tile to tile) and more workgroups asked
+# for than there are slabs.
+TILES_CASES = [(777, 64, 3, 1), (777, 128, 3, 64), (777, 320, 2, 65), (2577, 192, 16, 128), (1000, 2560, 4, 100),
+               (50, 384, 256, 33), (41001, 320, 256, 17)]
+
+
+def tiles(grid):
+    return SkConfig.make(SK_PATH_STREAM, waves=8, ku=2, rows=160, split=1, grid=grid, groups=4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,Kd,grid,M", TILES_CASES)
+def test_stream_persistent_tiles(N, Kd, grid, M):
+    g = torch.Generator().manual_seed(N + Kd + M)
+    w, x = randn_bf16((N, Kd), 0.02, g), randn_bf16((M, Kd), 1.0, g)
+    wide = torch.full((N, Kd + 40), float("nan"), dtype=BF16, device=DEV)
+    wide[:, :Kd] = w.to(DEV)
+    xd = torch.full((M, Kd + 24), float("nan"), dtype=BF16, device=DEV)[:, :Kd]
+    xd.copy_(x)
+    ref = from_bits(oracle.gemm(bits(x), bits(w)))
+    for pad in (0, 3):   # 8-byte aligned output rows or not (with an odd N)
+        out = torch.full((M, (N + 7) // 4 * 4 + pad), float("nan"), dtype=BF16, device=DEV)
+        K.gemm(xd, wide[:, :Kd], out=out[:, :N], config=tiles(grid))
+        torch.cuda.synchronize()
+        assert_parity(out[:, :N], ref, f"N={N} K={Kd} grid={grid} M={M}")
+        assert torch.isnan(out[:, N:]).all()
+    # the fused argmax: of this kernel's own logits, the lowest index of ties
+    ws = K._workspace(K.SK_OP_LM_ARGMAX, M, N, Kd, tiles(grid), DEV)
+    for _ in range(2):
+        ids, maxv = K.lm_argmax(xd, wide[:, :Kd], config=tiles(grid), ws=ws)
+        logits = out[:, :N].float()
+        best = logits.max(-1).values
+        first = (logits == best[:, None]).float().argmax(-1)
+        assert torch.equal(maxv, best) and torch.equal(ids, first)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,Kd,M", [(40960, 320, 33), (41000, 128, 64), (45001, 640, 65), (40960, 192, 130)])
+def test_default_routes_of_many_weight_rows(N, Kd, M):
+    g = torch.Generator().manual_seed(N + M)
+    w, x = randn_bf16((N, Kd), 0.02, g).to(DEV), randn_bf16((M, Kd), 1.0, g).to(DEV)
+    mm = K.SkinnyMatmul(M, N, Kd, DEV)
+    out = mm(x, w)
+    assert_parity(out, (x.float() @ w.float().t()).cpu(), "fp32 product")
+    am = K.LmArgmax(M, N, Kd, DEV)
+    ids, maxv = am(x, w)
+    ids, maxv = ids.clone(), maxv.clone()
+    best = out.float().max(-1).values
+    assert torch.equal(maxv[:128], best[:128])
+    assert torch.equal(ids[:128], (out[:128].float() == best[:128, None]).float().argmax(-1))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        mm(x, w), am(x, w)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        c_out, (c_ids, c_max) = mm(x, w), am(x, w)
+    for _ in range(3):
+        c_out.zero_(), c_ids.zero_(), c_max.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c_out, out) and torch.equal(c_ids, ids) and torch.equal(c_max, maxv)
+
+
 # Calls without a configuration take the stream plan that their workspace
 # allows: every route of a shape against the oracle, also replayed from a graph.
 ROUTES = [(6144, 2560, m) for m in (2, 16, 17, 48, 49, 64, 65, 128, 130)] + \
@@ -160,6 +228,10 @@ def test_stream_configs_are_planned():
     assert ok(stream(40, 2), K.SK_OP_GATEUP, N=9728) == SK_ERR_CONFIG
     assert ok(stream(24), K.SK_OP_RESID_GEMM) == SK_ERR_CONFIG    # 24: not whole 16-column groups
     assert ok(stream(32), K.SK_OP_PRE_GEMM) == SK_ERR_CONFIG
+    assert ok(tiles(256)) == SK_OK and ok(tiles(256), K.SK_OP_LM_ARGMAX) == SK_OK
+    assert ok(tiles(256), Kd=2592) == SK_ERR_CONFIG
+    for op in (K.SK_OP_GATEUP, K.SK_OP_RESID_GEMM, K.SK_OP_PRE_GEMM):   # logits and argmax only
+        assert ok(tiles(256), op) == SK_ERR_CONFIG
     # counters (one per tile, padded to 256 bytes), then a block per tile and split
     assert _lib.workspace_bytes(K.SK_OP_GEMM, 16, 2560, 9728, stream(32, 3)) == 512 + 80 * 3 * 16 * 32 * 4
     assert _lib.workspace_bytes(K.SK_OP_GEMM, 5, 777, 2560, stream(10, 2)) == 512 + 78 * 2 * 5 * 12 * 4
