@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 #include <string.h>
 #include <unordered_map>
@@ -421,8 +422,12 @@ int grid_bound(const Plan& pl) {
 }
 
 // Workspace layout: [arrival counters, padded to 256 B][partials or argmax
-// candidates].  The counters must be zero before the first call (allocate the
-// workspace zero-filled); every call returns them to zero.
+// candidates][normalised rows of a separate norm launch].  The counters must be
+// zero before the first call (allocate the workspace zero-filled); every call
+// returns them to zero.  A workspace serves plans with different numbers of
+// counters (the launches of one call, the default plan and the stream plans of
+// a shape), so ticket_min widens the counter area of each to the widest:
+// nothing that one of them writes lies where another expects zeros.
 size_t ticket_bytes(int n) { return (((size_t)n * sizeof(unsigned)) + 255) & ~(size_t)255; }
 
 // With row groups: one counter (argmax) or one per tile for each group, the
@@ -431,6 +436,7 @@ size_t plan_tickets(int op, const Plan& pl) {
   const size_t n = ticket_bytes(pl.groups * (base_op(op) == SK_OP_LM_ARGMAX ? 1 : pl.nrb));
   return n > pl.ticket_min ? n : pl.ticket_min;
 }
+bool uses_counters(int op, const Plan& pl) { return pl.cfg.split > 1 || base_op(op) == SK_OP_LM_ARGMAX; }
 size_t plan_workspace(int op, int M, int N, const Plan& pl) {
   op = base_op(op);
   if (op == SK_OP_LM_ARGMAX) return plan_tickets(op, pl) + (size_t)M * sizeof(unsigned long long);
@@ -631,6 +637,15 @@ const StreamEntry* stream_lookup(int op, int M, int N, int K, int n) {
   for (const StreamEntry& e : kStream)
     if (e.op == op && e.N == N && e.K == K && e.m_lo <= M && M <= e.m_hi && n-- == 0) return &e;
   return nullptr;
+}
+
+// Counter bytes of the widest stream plan of op/N/K, whatever its rows (0: none
+// has counters).
+size_t stream_counters(int op, int N, int K) {
+  size_t n = 0;
+  for (const StreamEntry& e : kStream)
+    if (e.op == op && e.N == N && e.K == K && e.cfg.split > 1) n = std::max(n, ticket_bytes(cdiv(N, e.cfg.rows)));
+  return n;
 }
 
 // The stream kernels address a tile's rows with 32-bit byte offsets.
@@ -890,13 +905,15 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 // Plans of one call: rows beyond one launch's (launch_rows) are processed in
 // chunks of that many rows (each streaming the weights once more), so a call
 // has at most two distinct chunk sizes.  Also the workspace it needs: the
-// plans' counters and partials, then, when the norm prologue runs as its own
-// launch, the normalised activations [M, K] at offset `norm_off`.
+// plans' counters (`counters` bytes, all plans of the shape included) and
+// partials, then, when the norm prologue runs as its own launch, the normalised
+// activations [M, K] at offset `norm_off`.
 struct CallPlan {
   Plan plans[2];
   int chunk = 0;                // rows per launch
   int chunk_rows[2] = {0, 0};
   int nplans = 0;
+  size_t counters = 0;
   size_t base_need = 0;
   size_t norm_off = 0;
   size_t need = 0;
@@ -914,6 +931,21 @@ int launch_rows(int op, int M, int N, int K, const sk_config* cfg) {
       plan_shape(op, R, N, K, c, &pl) == SK_OK)
     return kMaxLaunchM;
   return kMaxM;
+}
+
+// The workspace of cp's plans behind its counter area.
+void lay_out(int op, int M, int N, int K, CallPlan* cp) {
+  cp->base_need = 0;
+  for (int i = 0; i < cp->nplans; ++i) {
+    Plan& pl = cp->plans[i];
+    pl.ticket_min = uses_counters(op, pl) ? cp->counters : 0;
+    cp->base_need = std::max(cp->base_need, plan_workspace(op, cp->chunk_rows[i], N, pl));
+  }
+  cp->need = cp->base_need;
+  if (is_norm_op(op) && !cp->fused) {
+    cp->norm_off = align256(std::max(cp->base_need, cp->counters));
+    cp->need = cp->norm_off + (size_t)M * K * sizeof(sk_bf16);
+  }
 }
 
 int plan_call(int op, int M, int N, int K, const sk_config* cfg, CallPlan* cp) {
@@ -949,47 +981,40 @@ int plan_call(int op, int M, int N, int K, const sk_config* cfg, CallPlan* cp) {
       cp->plans[i].norm = true;
     }
   }
-  cp->base_need = 0;
-  for (int i = 0; i < cp->nplans; ++i) {
-    const size_t n = plan_workspace(op, cp->chunk_rows[i], N, cp->plans[i]);
-    if (n > cp->base_need) cp->base_need = n;
-  }
-  cp->need = cp->base_need;
-  if (is_norm_op(op) && !cp->fused) {
-    cp->norm_off = align256(cp->base_need);
-    cp->need = cp->norm_off + (size_t)M * K * sizeof(sk_bf16);
-  }
+  cp->counters = cp->fused ? 0 : stream_counters(base_op(op), N, K);
+  for (int i = 0; i < cp->nplans; ++i)
+    if (uses_counters(op, cp->plans[i])) cp->counters = std::max(cp->counters, plan_tickets(op, cp->plans[i]));
+  // The remainder of a call without a configuration has a plan of its own; the
+  // default configuration passed explicitly shares its workspace all the same.
+  CallPlan def;
+  if (cp->nplans == 2 && !cp->fused && cfg && cfg->path != SK_PATH_AUTO &&
+      plan_call(op, M, N, K, nullptr, &def) == SK_OK && !def.fused)
+    cp->counters = std::max(cp->counters, def.counters);
+  lay_out(op, M, N, K, cp);
   return SK_OK;
 }
 
 // The call with stream-path plans in place of cp's, taking the n-th entry of
 // each launch's rows where there is one; false when no launch has an n-th
-// entry.  The counters of both plans lie inside one area, so calls with and
-// without a configuration can share a workspace.
+// entry.  cp's counter area covers these plans too, so one workspace serves
+// them and cp's own, whichever a call takes (by its configuration, its strides
+// or the workspace's size).
 bool stream_call(int op, int M, int N, int K, const CallPlan& cp, int n, CallPlan* out) {
   if (cp.fused) return false;
   const int bop = base_op(op);
   *out = cp;
   bool any = false;
-  out->base_need = 0;
   for (int i = 0; i < cp.nplans; ++i) {
     if (const StreamEntry* e = stream_lookup(bop, cp.chunk_rows[i], N, K, n)) {
       Plan pl;
       if (plan_shape_impl(bop, cp.chunk_rows[i], N, K, e->cfg, false, &pl) == SK_OK) {
-        if (cp.plans[i].cfg.split > 1) pl.ticket_min = plan_tickets(bop, cp.plans[i]);
         pl.norm = cp.plans[i].norm;
         out->plans[i] = pl;
         any = true;
       }
     }
-    const size_t need = plan_workspace(bop, cp.chunk_rows[i], N, out->plans[i]);
-    if (need > out->base_need) out->base_need = need;
   }
-  out->need = out->base_need;
-  if (is_norm_op(op)) {
-    out->norm_off = align256(out->base_need);
-    out->need = out->norm_off + (size_t)M * K * sizeof(sk_bf16);
-  }
+  lay_out(op, M, N, K, out);
   return any;
 }
 
@@ -1191,14 +1216,17 @@ int plan_handoff(int op, int M, int N, int K, const sk_config* cfg, Plan* pl) {
   sk_config c;
   int st = handoff_config(op, M, N, K, cfg, &c);
   if (st) return st;
-  return plan_shape_impl(handoff_base(op), M, N, K, c, false, pl, handoff_variant(op));
+  st = plan_shape_impl(handoff_base(op), M, N, K, c, false, pl, handoff_variant(op));
+  if (st == SK_OK && uses_counters(handoff_base(op), *pl)) pl->ticket_min = stream_counters(op, N, K);
+  return st;
 }
 
 // The n-th stream plan of a hand-off op in place of pl (its default plan).
 bool stream_handoff(int op, int M, int N, int K, const Plan& def, int n, Plan* pl) {
   const StreamEntry* e = stream_lookup(op, M, N, K, n);
   if (!e || plan_shape_impl(handoff_base(op), M, N, K, e->cfg, false, pl, handoff_variant(op)) != SK_OK) return false;
-  if (def.cfg.split > 1) pl->ticket_min = plan_tickets(handoff_base(op), def);
+  pl->ticket_min = stream_counters(op, N, K);
+  if (def.cfg.split > 1) pl->ticket_min = std::max(pl->ticket_min, plan_tickets(handoff_base(op), def));
   return true;
 }
 

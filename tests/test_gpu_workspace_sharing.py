@@ -1,0 +1,86 @@
+"""One workspace under every plan that calls of a shape may take.
+
+A call's plan depends on its configuration, its strides and the workspace's
+size, and past 128 rows a call has two launches with plans of their own.  The
+arrival counters of all of them lie at the workspace's start, where every call
+leaves zeros, so nothing that one plan writes (split-K partials, the normalised
+rows of a separate norm launch) may lie below the counters of another.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import oracle
+from starter_amd import _lib
+from starter_amd import kernels as K
+from tests._util import BF16, assert_parity, bits, from_bits, randn_bf16
+
+DEV = "cuda:0"
+COUNTERS = 512   # 80 tiles of 32 rows, 4 bytes each, padded to 256: the stream plans of 2560 columns
+
+
+@pytest.mark.parametrize("N,Kd,ms", [(2560, 4096, (16, 17, 32, 64, 65, 96)), (2560, 9728, (3, 8, 16))])
+def test_norm_rows_lie_behind_the_stream_plans_counters(N, Kd, ms):
+    """Unsplit default plans: no counters of their own, but the norm launch's
+    rows stay clear of those of the stream plans (any row count's)."""
+    for M in ms:
+        assert _lib.workspace_bytes(K.SK_OP_GEMM, M, N, Kd) == 0
+        assert _lib.workspace_bytes(K.SK_OP_RMSNORM_GEMM, M, N, Kd) == COUNTERS + 2 * M * Kd, M
+
+
+def test_launches_of_one_call_share_a_counter_area():
+    """Down at 161 rows: 128 rows in 80 tiles and three splits, then 33 in 160
+    tiles and four; the first launch's partials start behind both."""
+    assert _lib.workspace_bytes(K.SK_OP_GEMM, 128, 2560, 9728) == 512 + 3 * 128 * 2560 * 4
+    assert _lib.workspace_bytes(K.SK_OP_GEMM, 161, 2560, 9728) == 768 + 3 * 128 * 2560 * 4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,Kd,M", [(2560, 4096, 17), (2560, 4096, 64), (2560, 9728, 8)])
+def test_normed_calls_share_a_workspace(N, Kd, M):
+    """Stream plan (split K), the default plan passed explicitly (norm rows in
+    the workspace, no split) and a smaller call without a configuration, then
+    the stream plan again: its counters are still zero."""
+    g = torch.Generator().manual_seed(N + Kd + M)
+    x, y, w = (randn_bf16(s, c, g).to(DEV) for s, c in (((M, Kd), 1.0), ((M, Kd), 1.0), ((N, Kd), 0.02)))
+    gain = (1 + 0.1 * torch.randn(Kd, generator=g)).to(BF16).to(DEV)
+    xo = torch.empty_like(x)
+    ws = torch.zeros(_lib.workspace_bytes_preferred(K.SK_OP_RMSNORM_GEMM, M, N, Kd), dtype=torch.uint8, device=DEV)
+
+    def call(rows=M, config=None):
+        out = torch.full((rows, N), float("nan"), dtype=BF16, device=DEV)
+        return K.rmsnorm_gemm(x[:rows], y[:rows], gain, 1e-6, xo[:rows], w, out=out, config=config, ws=ws)
+
+    first = call()
+    h = xo.double()
+    h = h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + 1e-6) * gain.double()
+    want = (h @ w.double().t()).float()
+    # bf16 rounding of the norm's two steps and of the output, all relative: 3 * 2^-9 on each term of the sum
+    assert ((first.float() - want).norm() / want.norm()).item() < 3 * 2.0 ** -9
+    assert not bool(ws[:COUNTERS].any())
+    explicit = call(config=_lib.default_config(K.SK_OP_RMSNORM_GEMM, M, N, Kd))
+    assert not bool(ws[:COUNTERS].any())
+    assert ((explicit.float() - want).norm() / want.norm()).item() < 3 * 2.0 ** -9
+    assert torch.equal(call().view(torch.int16), first.view(torch.int16))
+    call(rows=2)
+    assert not bool(ws[:COUNTERS].any())
+    assert torch.equal(call().view(torch.int16), first.view(torch.int16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [129, 161, 176, 255])
+def test_launches_past_128_rows(M):
+    """Two launches with different plans on one workspace, twice."""
+    N, Kd = 2560, 9728
+    g = torch.Generator().manual_seed(M)
+    x, w = randn_bf16((M, Kd), 1.0, g), randn_bf16((N, Kd), 0.02, g)
+    ref = from_bits(oracle.gemm(bits(x), bits(w)))
+    xd, wd = x.to(DEV), w.to(DEV)
+    for n in (_lib.workspace_bytes(K.SK_OP_GEMM, M, N, Kd), _lib.workspace_bytes_preferred(K.SK_OP_GEMM, M, N, Kd)):
+        ws = torch.zeros(n, dtype=torch.uint8, device=DEV)
+        for _ in range(2):
+            out = torch.full((M, N), float("nan"), dtype=BF16, device=DEV)
+            assert_parity(K.gemm(xd, wd, out=out, ws=ws), ref, f"M={M} workspace {n}")
+            assert not bool(ws[:512].any())
