@@ -1510,8 +1510,7 @@ int sk_swiglu_bf16(const sk_bf16* gu, int64_t ld_gu, sk_bf16* out, int64_t ld_ou
   int st = device_info(&num_cu);
   if (st) return st;
   if (I % 8 == 0 && ((ld_gu | ld_out) & 7) == 0 && aligned16(gu) && aligned16(out)) {
-    const int rb = cdiv(M, sk::SWIGLU_ROWS);
-    sk::swiglu_vec_kernel<<<dim3((unsigned)cdiv(I, 8 * 256), (unsigned)(rb < 65535 ? rb : 65535)), dim3(256), 0,
+    sk::swiglu_vec_kernel<<<dim3((unsigned)cdiv(I, 8 * 256), (unsigned)(M < 65535 ? M : 65535)), dim3(256), 0,
                             stream>>>(gu, ld_gu, out, ld_out, M, I);
     return launch_status();
   }

@@ -1594,32 +1594,25 @@ __global__ void __launch_bounds__(256) clear_words_kernel(unsigned* __restrict__
 
 // Unfused SwiGLU over gu = [g | u] (engine/kernels/swiglu.py:14-24), eight
 // columns per thread: rows of 8-column multiples whose base and strides are
-// 16-byte aligned.  Workgroup (column block, row block); a thread loads its
-// columns of SWIGLU_ROWS rows before it uses any.  Bound by memory: 16384 rows
-// x 9728 (956 MB) 171-185 us, 5.2-5.6 TB/s, where 2-byte accesses took 284-294.
-constexpr int SWIGLU_ROWS = 4;
+// 16-byte aligned.  Workgroup (column block, row).  Bound by memory from some
+// hundred rows on: 16384 rows x 9728 (956 MB) 175 us, 5.5 TB/s, where 2-byte
+// accesses take 280; below, by the launch and one thread's chain of loads and
+// exponentials.  So a thread takes one row: with four rows each (and a quarter
+// of the workgroups) the chain took 4.7 us at 4-64 rows x 9728 where one row
+// takes 2.7-3.2 and 2-byte accesses 2.6-4.0, and 180 us at 16384.
 __global__ void __launch_bounds__(256) swiglu_vec_kernel(const uint16_t* __restrict__ gu, int64_t ld_gu,
                                                          uint16_t* __restrict__ out, int64_t ld_out, int M, int I) {
   const int i = 8 * (blockIdx.x * 256 + threadIdx.x);
   if (i >= I) return;
-  for (int m0 = blockIdx.y * SWIGLU_ROWS; m0 < M; m0 += gridDim.y * SWIGLU_ROWS) {
-    u32x4 g[SWIGLU_ROWS], u[SWIGLU_ROWS];
+  for (int m = blockIdx.y; m < M; m += gridDim.y) {
+    const uint16_t* row = gu + (int64_t)m * ld_gu + i;
+    const u32x4 g = ld16_stream(row), u = ld16_stream(row + I);
+    u32x4 y;
 #pragma unroll
-    for (int k = 0; k < SWIGLU_ROWS; ++k) {
-      const uint16_t* row = gu + (int64_t)min(m0 + k, M - 1) * ld_gu + i;
-      g[k] = ld16_stream(row);
-      u[k] = ld16_stream(row + I);
-    }
-#pragma unroll
-    for (int k = 0; k < SWIGLU_ROWS; ++k) {
-      if (m0 + k >= M) break;
-      u32x4 y;
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        y[q] = (uint32_t)swiglu_bf(bf2f(g[k][q] & 0xFFFFu), bf2f(u[k][q] & 0xFFFFu)) |
-               ((uint32_t)swiglu_bf(bf2f(g[k][q] >> 16), bf2f(u[k][q] >> 16)) << 16);
-      *reinterpret_cast<u32x4*>(out + (int64_t)(m0 + k) * ld_out + i) = y;
-    }
+    for (int q = 0; q < 4; ++q)
+      y[q] = (uint32_t)swiglu_bf(bf2f(g[q] & 0xFFFFu), bf2f(u[q] & 0xFFFFu)) |
+             ((uint32_t)swiglu_bf(bf2f(g[q] >> 16), bf2f(u[q] >> 16)) << 16);
+    *reinterpret_cast<u32x4*>(out + (int64_t)m * ld_out + i) = y;
   }
 }
 
