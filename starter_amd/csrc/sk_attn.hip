@@ -388,18 +388,35 @@ __global__ void __launch_bounds__(64 * ATTN_WAVES, 4) decode_attn_kernel(AttnArg
   };
   const std::false_type keys{};
   const std::true_type values{};
-  // The first block is on its way while the query rows are formed, unless it
-  // holds rows that this launch writes (the caches below pos are not written).
+  const int r16 = lane & 15;
+  const int my_gr = rbk * QR + r16;
+  const bool my_real = r16 < QR && my_gr < rows;
+  const int my_t = my_gr / a.G;
+  // (requested before any key, so that nothing waits for it behind those)
+  long long my_tree = 0ll;
+  if constexpr (TREE) my_tree = my_real ? (long long)a.tree[min(my_t, a.R - 1)] : 0ll;
+  // The first block's keys are on their way while the query rows are formed,
+  // unless it holds rows that this launch writes (the caches below pos are not
+  // written).  Not its values: loads return in order, so everything the query
+  // rows need would wait behind them too (with the values: 16 sequences of 300
+  // keys, one row, 9.2 us, without 9.0; 64 of up to 200 12.0 and 11.5; 32 x 4
+  // tree rows of up to 500 15.6 and 15.2; 5 x 8 of up to 1000 13.5 and 13.1).
   const bool early = nblk > 0 && wk0 + 16 <= min(end, pos);   // (uniform)
-  if (early) {
-    issue(0, keys);
-    issue(0, values);
-  }
+  if (early) issue(0, keys);
+  // (ancestor masks wait in LDS for the few masked blocks; every wave stores the
+  // same values and reads them back itself, in order)
+  __shared__ long long s_tree[TREE ? QR : 1];
+  auto issue_rest = [&]() {
+    if (TREE && r16 < QR) s_tree[r16] = my_tree;
+    if (nblk > 0) {
+      if (!early) issue(0, keys);
+      issue(0, values);
+    }
+  };
 
   // Query rows r = t*G + g (head kh*G + g, query row t) as the B operand of
   // v_mfma_f32_16x16x32_bf16: lane l supplies row l%16, dims 32s + 8*(l/16)
   // for K step s (rows >= QR are zero columns).
-  const int r16 = lane & 15;
   bf16x8 qb[HEAD_D / 32];
   if constexpr (ROPE) {
     // Query rows through the norm + rotary step (one wave per row), into LDS.
@@ -446,6 +463,7 @@ __global__ void __launch_bounds__(64 * ATTN_WAVES, 4) decode_attn_kernel(AttnArg
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
+    issue_rest();
     const bool real = r16 < QR;
 #pragma unroll
     for (int st = 0; st < HEAD_D / 32; ++st) {
@@ -463,22 +481,14 @@ __global__ void __launch_bounds__(64 * ATTN_WAVES, 4) decode_attn_kernel(AttnArg
       const u32x4 v = ld16(qp + 32 * st);
       qb[st] = __builtin_bit_cast(bf16x8, real ? v : u32x4{0u, 0u, 0u, 0u});
     }
+    issue_rest();
   }
   // Lane l owns query row l%16 (its MFMA column) and, in each 16-key block,
   // keys 4*(l/16) .. +3 of that row; the 4 lanes of a row share its running
   // max and keep partial sums.  acc[c][k] = O[row l%16][dim 8*(4*(l/16)+k) + c].
   // Visibility of key n to the row: keys before pos always; key pos + j
   // (j < R) iff j <= t (chain) or bit j of tree[t] is set (draft tree).
-  const int my_gr = rbk * QR + r16;
-  const bool my_real = r16 < QR && my_gr < rows;
-  const int my_t = my_gr / a.G;
   const int row_lim = my_real ? pos + my_t : -1;   // last visible key of the row (chain)
-  // (ancestor masks wait in LDS for the few masked blocks; every wave stores the
-  // same values and reads them back itself, in order)
-  __shared__ long long s_tree[TREE ? QR : 1];
-  if constexpr (TREE) {
-    if (r16 < QR) s_tree[r16] = my_real ? (long long)a.tree[min(my_t, a.R - 1)] : 0ll;
-  }
 
   float m = -INFINITY, l = 0.f;
   f32x4 acc[8];
@@ -530,10 +540,6 @@ __global__ void __launch_bounds__(64 * ATTN_WAVES, 4) decode_attn_kernel(AttnArg
     m = mx;
   };
   const int unmasked_end = min(end, pos);   // keys below it need no masks
-  if (nblk > 0 && !early) {
-    issue(0, keys);
-    issue(0, values);
-  }
   for (int i = 0; i < nblk; ++i) {
     const bool more = i + 1 < nblk;
     const int n0 = wk0 + 16 * ATTN_WAVES * i;
