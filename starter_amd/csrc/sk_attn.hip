@@ -726,8 +726,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 int cdiv(int a, int b) { return (a + b - 1) / b; }
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-// Waves per workgroup, 16 keys each per block (at B = 16, ~1.1k keys, one
-// split: 8 waves 15.4 us, 4 waves 15.9 us).
+// Waves per workgroup, 16 keys each per block.
 constexpr int kAttnWaves = 8;
 
 struct AttnPlan {
@@ -735,9 +734,10 @@ struct AttnPlan {
   size_t tickets = 0, part_o = 0, part_ml = 0, need = 0;
 };
 
-// Splits: the keys of one (b, kv head) pair are split when B*HKV alone
-// leaves most compute units idle, each split a whole number of workgroup
-// blocks (16 keys per wave) of the longest sequence the plan will see.
+// S: the most key ranges of a (sequence, KV head) pair (the kernel cuts them
+// from each sequence's length: key_range), no more than the planned length has
+// workgroup blocks (16 keys per wave).  split_len: the planned length over S,
+// in whole blocks; S of them are the keys the plan covers.
 int attn_plan(int B, int HQ, int HKV, int D, int R, int cap, int max_len, int nsplit, AttnPlan* p) {
   if (B < 1 || HKV < 1 || HQ < HKV || HQ % HKV != 0 || R < 1 || cap < 1 || D != sk::HEAD_D) return SK_ERR_SHAPE;
   const int G = HQ / HKV;
@@ -755,14 +755,19 @@ int attn_plan(int B, int HQ, int HKV, int D, int R, int cap, int max_len, int ns
   const int blocks = cdiv(work, block);
   int S = nsplit;
   if (S <= 0) {
-    // Decode (one query row per sequence): about one workgroup per CU of an
-    // MI355X (B = 16, 8 KV heads, 1089 keys: 17.4 us in one split per pair,
-    // 16.8 in two; B = 4: 10.9 -> 9.6 us; decode step 5896 -> 5978 tok/s).
-    // Verify rows (R > 1, one or more 16-row blocks per pair): about one per
-    // two CUs, where a second split cost the 16 x 8 verify pass 10%.
-    const long pairs = (long)B * HKV;
+    // One query row: about one workgroup per CU (256; 16 x 2000 keys in one
+    // range 28.7 us, in two 25.1, in three 26.1, in four 24.7).  Verify rows
+    // (R > 1): half of that (16 x 8 rows of up to 1000 keys in one range 18.9
+    // us, in two 22.3; 16 x 2 rows 17.9 and 17.2).
+    const long pairs = (long)B * HKV, groups = pairs * p->NRB;
     const long target = R == 1 ? 256 : 128;
     S = (int)((target + pairs - 1) / pairs);
+    // Between one workgroup per CU and two, some CUs hold two and the rest wait
+    // for them; then only as many ranges as fit the CUs once.  3 x 16000 keys
+    // 45.0 us in 11 ranges (264 workgroups), 35.3 in 10 (240); 12 x 4000 42.4
+    // in 3 (288), 34.2 in 2 (192); 6 x 8 tree rows of up to 4000 35.3 in 3 (two
+    // row blocks each, 288), 29.3 in 2 (192).
+    if (groups * S > 256 && groups * S < 512) S = (int)(256 / groups);
     if (S > 32) S = 32;
   }
   if (S > blocks) S = blocks;

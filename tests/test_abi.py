@@ -610,3 +610,22 @@ def test_rope_and_attention_parameters_are_checked_before_launch():
             K._vec(t, "pos", torch.int32, n, exact=exact)
     with pytest.raises(ValueError, match="device"):
         K._vec(torch.zeros(4, dtype=torch.int32), "pos", torch.int32, 4, exact=False)   # right shape, host memory
+
+
+@pytest.mark.parametrize("R", [1, 2, 4, 8, 16])
+def test_attention_plans_fill_the_compute_units_evenly(R):
+    """Key ranges of a plan: never a launch of more workgroups than CUs (256)
+    but fewer than two for each (264 keep the chip busy about as long as 512),
+    unless one range of each (sequence, KV head, row block) makes it one."""
+    HQ, HKV, cap = 32, 8, 32768
+    rows = HQ // HKV * R
+    qr = 4 if rows <= 4 else 8 if rows <= 8 else 16
+    blocks = -(-rows // qr)
+    for B in range(1, 65):
+        groups = B * HKV * blocks
+        need = _lib.lib().sk_decode_attention_workspace_bytes(B, HQ, HKV, 128, R, cap, cap, 0)
+        per = groups * qr * (128 + 2) * 4     # a range's partial rows, maxima and sums
+        ranges = round((need - _tickets(groups)) / per) if need else 1
+        assert need == 0 or need == _tickets(groups) + ranges * per, B
+        assert ranges == 1 or groups * ranges <= 256 or groups * ranges >= 512, (B, ranges)
+        assert 1 <= ranges <= 32 and (ranges == 32 or 2 * groups * ranges > 128), (B, ranges)
