@@ -86,7 +86,10 @@ typedef enum sk_path {
  * Launch configuration.  The reference picks a Triton config per shape at
  * warmup (engine/kernels/gemm.py:381-401, 516-558); here the defaults come
  * from an offline-tuned table (sk_default_config) and an explicit config can
- * be passed to any op (NULL = default) to test or time one candidate.
+ * be passed to any op to test or time one candidate.  NULL (or SK_PATH_AUTO)
+ * is not the same as passing sk_default_config's result: at most of the tuned
+ * shapes such a call takes a plan of the stream path where its workspace holds
+ * it (sk_workspace_bytes_preferred; sk_selected_config names the plan).
  *
  *   path   : SK_PATH_MFMA, SK_PATH_MFMA_LDS, SK_PATH_GEMV, SK_PATH_WIDE or
  *            SK_PATH_STREAM
@@ -169,8 +172,10 @@ int sk_version(void);
 /* Static message for a status code. */
 const char* sk_strerror(int status);
 
-/* Default launch configuration for op at (M, N, K) on a device with num_cu
- * compute units (pass 0 for the MI355X's 256).  Pure host logic.
+/* Launch configuration of the table for op at (M, N, K) on a device with num_cu
+ * compute units (pass 0 for the MI355X's 256): the plan of the least workspace,
+ * which sk_workspace_bytes reports, never a stream plan (see
+ * sk_selected_config).  Pure host logic.
  * Replaces the warmup-time pickers pick_matmul / pick_gateup / pick_normed
  * (engine/kernels/gemm.py:516-660). */
 int sk_default_config(int op, int M, int N, int K, int num_cu, sk_config* out);
@@ -189,6 +194,12 @@ size_t sk_workspace_bytes(int op, int M, int N, int K, const sk_config* cfg);
  * sk_workspace_bytes, which is the least that any call needs.  Zero-filled
  * once like every workspace; the plan depends only on op, shape and ws_bytes. */
 size_t sk_workspace_bytes_preferred(int op, int M, int N, int K);
+
+/* The configuration of the plan that a call without one takes with a workspace
+ * of ws_bytes (past 128 rows that of its first launch; row strides whose tiles
+ * span 2 GiB fall back on sk_default_config's).  Pure host logic; SK_ERR_WORKSPACE
+ * when ws_bytes is less than sk_workspace_bytes. */
+int sk_selected_config(int op, int M, int N, int K, size_t ws_bytes, sk_config* out);
 
 /* C[M,N] = bf16(A[M,K] @ W[N,K]^T), fp32 accumulation.
  * Replaces SkinnyMatmul.__call__ / _skinny_kernel + _sum_kernel

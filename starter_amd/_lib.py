@@ -49,7 +49,7 @@ SK_PATH_STREAM = 5
 # Every symbol include/starter_amd.h declares (checked by the CPU tests).
 EXPORTS = (
     "sk_version", "sk_strerror", "sk_default_config", "sk_check_config", "sk_workspace_bytes",
-    "sk_workspace_bytes_preferred",
+    "sk_workspace_bytes_preferred", "sk_selected_config",
     "sk_gemm_bf16", "sk_gemm_bf16_noalloc", "sk_gateup_swiglu_bf16", "sk_lm_argmax_bf16", "sk_argmax_bf16",
     "sk_add_rmsnorm_bf16", "sk_swiglu_bf16",
     "sk_rmsnorm_gemm_bf16", "sk_rmsnorm_gateup_swiglu_bf16", "sk_rmsnorm_lm_argmax_bf16",
@@ -109,6 +109,7 @@ _SIGNATURES = {
     "sk_check_config": (_i32, [_i32, _i32, _i32, _i32, _cfgp]),
     "sk_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _cfgp]),
     "sk_workspace_bytes_preferred": (_sz, [_i32, _i32, _i32, _i32]),
+    "sk_selected_config": (_i32, [_i32, _i32, _i32, _i32, _sz, _cfgp]),
     "sk_gemm_bf16": (_i32, [_p, _i64, _p, _i64, _p, _i64, _i32, _i32, _i32, _cfgp, _p, _sz, _p]),
     "sk_gemm_bf16_noalloc": (_i32, [_p, _i64, _p, _i64, _p, _i64, _i32, _i32, _i32, _cfgp, _p]),
     "sk_gateup_swiglu_bf16": (_i32, [_p, _i64, _p, _p, _i64, _p, _i64, _i32, _i32, _i32, _cfgp, _p, _sz, _p]),
@@ -198,3 +199,12 @@ def workspace_bytes_preferred(op: int, M: int, N: int, K: int) -> int:
     """Workspace with which calls without a configuration run their fastest
     plan (``workspace_bytes`` is the least they run with)."""
     return int(lib().sk_workspace_bytes_preferred(op, M, N, K))
+
+
+def selected_config(op: int, M: int, N: int, K: int, ws_bytes: int | None = None) -> SkConfig:
+    """The plan that a call without a configuration takes with ``ws_bytes`` of
+    workspace (default: ``workspace_bytes_preferred``)."""
+    c = SkConfig()
+    n = workspace_bytes_preferred(op, M, N, K) if ws_bytes is None else ws_bytes
+    check(lib().sk_selected_config(op, M, N, K, n, ctypes.byref(c)), "sk_selected_config")
+    return c

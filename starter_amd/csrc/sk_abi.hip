@@ -1018,6 +1018,19 @@ bool stream_call(int op, int M, int N, int K, const CallPlan& cp, int n, CallPla
   return any;
 }
 
+// The plans of a call without a configuration that has `avail` workspace bytes:
+// cp, or the first stream entry's that fit them.  False when not even cp fits.
+bool select_call(int op, int M, int N, int K, size_t avail, CallPlan* cp) {
+  if (cp->need > avail) return false;
+  CallPlan alt;
+  for (int n = 0; stream_call(op, M, N, K, *cp, n, &alt); ++n)
+    if (alt.need <= avail) {
+      *cp = alt;
+      break;
+    }
+  return true;
+}
+
 // Shared driver of the GEMM-family ops.  nrm != nullptr: A is x and the
 // projection consumes rmsnorm(x + y) (op is then a SK_OP_RMSNORM_* op).
 int run_gemm_family(int op, const sk_bf16* A, int64_t lda, const NormIn* nrm, const sk_bf16* W0, const sk_bf16* W1,
@@ -1053,16 +1066,11 @@ int run_gemm_family(int op, const sk_bf16* A, int64_t lda, const NormIn* nrm, co
   } else if (cp.need > 0 && (!ws || ws_bytes < cp.need)) {
     return SK_ERR_WORKSPACE;
   }
+  const bool strides_ok = stream_strides_ok(M, nrm ? K : lda, 256, ldw);
   if (!cfg || cfg->path == SK_PATH_AUTO) {
     // (the allocation-free call takes the plan that the least workspace gets)
-    const size_t avail = noalloc ? cp.need : (ws ? ws_bytes : 0);
-    CallPlan alt;
-    for (int n = 0; stream_call(op, M, N, K, cp, n, &alt); ++n) {
-      if (alt.need > avail) continue;
-      if (stream_strides_ok(M, nrm ? K : lda, 256, ldw)) cp = alt;
-      break;
-    }
-  } else if (cfg->path == SK_PATH_STREAM && !stream_strides_ok(M, nrm ? K : lda, 256, ldw)) {
+    if (strides_ok) select_call(op, M, N, K, noalloc ? cp.need : (ws ? ws_bytes : 0), &cp);
+  } else if (cfg->path == SK_PATH_STREAM && !strides_ok) {
     return SK_ERR_SHAPE;
   }
   int num_cu = 0;
@@ -1230,6 +1238,19 @@ bool stream_handoff(int op, int M, int N, int K, const Plan& def, int n, Plan* p
   return true;
 }
 
+// As select_call.
+bool select_handoff(int op, int M, int N, int K, size_t avail, Plan* pl) {
+  const int bop = handoff_base(op);
+  if (plan_workspace(bop, M, N, *pl) > avail) return false;
+  Plan alt;
+  for (int n = 0; stream_handoff(op, M, N, K, *pl, n, &alt); ++n)
+    if (plan_workspace(bop, M, N, alt) <= avail) {
+      *pl = alt;
+      break;
+    }
+  return true;
+}
+
 size_t handoff_workspace(int op, int M, int N, int K, const sk_config* cfg) {
   Plan pl;
   if (plan_handoff(op, M, N, K, cfg, &pl)) return 0;
@@ -1281,14 +1302,10 @@ int run_handoff(int op, const sk_bf16* A, int64_t lda, const Handoff& h, const s
   if (st) return st;
   const size_t need = plan_workspace(bop, M, N, pl);
   if (need > 0 && (!ws || ws_bytes < need)) return SK_ERR_WORKSPACE;
+  const bool strides_ok = stream_strides_ok(M, lda, 256, ldw);
   if (!cfg || cfg->path == SK_PATH_AUTO) {
-    Plan alt;
-    for (int n = 0; stream_handoff(op, M, N, K, pl, n, &alt); ++n) {
-      if (plan_workspace(bop, M, N, alt) > (ws ? ws_bytes : 0)) continue;
-      if (stream_strides_ok(M, lda, 256, ldw)) pl = alt;
-      break;
-    }
-  } else if (cfg->path == SK_PATH_STREAM && !stream_strides_ok(M, lda, 256, ldw)) {
+    if (strides_ok) select_handoff(op, M, N, K, ws ? ws_bytes : 0, &pl);
+  } else if (cfg->path == SK_PATH_STREAM && !strides_ok) {
     return SK_ERR_SHAPE;
   }
   int num_cu = 0;
@@ -1391,6 +1408,26 @@ size_t sk_workspace_bytes(int op, int M, int N, int K, const sk_config* cfg) {
   CallPlan cp;
   if (plan_call(op, M, N, K, cfg, &cp)) return 0;
   return cp.need;
+}
+
+int sk_selected_config(int op, int M, int N, int K, size_t ws_bytes, sk_config* out) {
+  if (!out) return SK_ERR_NULL;
+  if (M < 1) return SK_ERR_SHAPE;
+  if (is_handoff_op(op)) {
+    Plan pl;
+    const int st = plan_handoff(op, M, N, K, nullptr, &pl);
+    if (st) return st;
+    if (!select_handoff(op, M, N, K, ws_bytes, &pl)) return SK_ERR_WORKSPACE;
+    *out = pl.cfg;
+    return SK_OK;
+  }
+  if (!is_gemm_family(base_op(op))) return SK_ERR_CONFIG;
+  CallPlan cp;
+  const int st = plan_call(op, M, N, K, nullptr, &cp);
+  if (st) return st;
+  if (!select_call(op, M, N, K, ws_bytes, &cp)) return SK_ERR_WORKSPACE;
+  *out = cp.plans[0].cfg;
+  return SK_OK;
 }
 
 size_t sk_workspace_bytes_preferred(int op, int M, int N, int K) {

@@ -753,7 +753,7 @@ class LmArgmax(_Planned):
 
 def _log_choice(log, what: str, op: int, M: int, N: int, K: int) -> None:
     if log:
-        log(f"{what} M={M} N={N} K={K}: {_lib.default_config(op, M, N, K).as_dict()}")
+        log(f"{what} M={M} N={N} K={K}: {_lib.selected_config(op, M, N, K).as_dict()}")
 
 
 def pick_matmul(a: torch.Tensor, w: torch.Tensor, log=None, ws: list | None = None):
@@ -781,12 +781,12 @@ def pick_normed(kind: str, x: torch.Tensor, y: torch.Tensor, w_norm: torch.Tenso
     M, K = x.shape
     if kind == "matmul":
         mm = SkinnyMatmul(M, w.shape[0], K, x.device, normed=True)
-        _log_choice(log, "normed matmul", SK_OP_GEMM, M, w.shape[0], K)
+        _log_choice(log, "normed matmul", SK_OP_RMSNORM_GEMM, M, w.shape[0], K)
         return lambda x, y, w_norm, xout, w: mm(x, w, norm=(y, w_norm, xout, eps))
     if kind == "gateup":
         I = w.shape[0] // 2
         mm = SkinnyGateUp(M, I, K, x.device, normed=True)
-        _log_choice(log, "normed gateup", SK_OP_GATEUP, M, I, K)
+        _log_choice(log, "normed gateup", SK_OP_RMSNORM_GATEUP, M, I, K)
         return lambda x, y, w_norm, xout, w: mm(x, w[:I], w[I:], norm=(y, w_norm, xout, eps))
     raise ValueError(f"unknown kind {kind!r}")
 
@@ -796,5 +796,5 @@ def pick_lm_argmax(x: torch.Tensor, w: torch.Tensor, eps: float, log=None):
     greedy argmax fused in (replaces ``mm["lm"](...).argmax(-1)``)."""
     M, K = x.shape
     mm = LmArgmax(M, w.shape[0], K, x.device, normed=True)
-    _log_choice(log, "normed lm_argmax", SK_OP_LM_ARGMAX, M, w.shape[0], K)
+    _log_choice(log, "normed lm_argmax", SK_OP_RMSNORM_LM_ARGMAX, M, w.shape[0], K)
     return lambda x, y, w_norm, xout, w: mm(x, w, norm=(y, w_norm, xout, eps))
