@@ -1431,18 +1431,18 @@ int sk_selected_config(int op, int M, int N, int K, size_t ws_bytes, sk_config* 
 }
 
 size_t sk_workspace_bytes_preferred(int op, int M, int N, int K) {
-  const size_t least = sk_workspace_bytes(op, M, N, K, nullptr);
-  if (M < 1) return least;
-  size_t want = 0;
+  if (M < 1) return 0;
   if (is_handoff_op(op)) {
     Plan def, pl;
-    if (plan_handoff(op, M, N, K, nullptr, &def) == SK_OK && stream_handoff(op, M, N, K, def, 0, &pl))
-      want = plan_workspace(handoff_base(op), M, N, pl);
-  } else if (is_gemm_family(base_op(op))) {
-    CallPlan cp, alt;
-    if (plan_call(op, M, N, K, nullptr, &cp) == SK_OK && stream_call(op, M, N, K, cp, 0, &alt)) want = alt.need;
+    if (plan_handoff(op, M, N, K, nullptr, &def)) return 0;
+    const size_t least = plan_workspace(handoff_base(op), M, N, def);
+    return stream_handoff(op, M, N, K, def, 0, &pl) ? std::max(least, plan_workspace(handoff_base(op), M, N, pl))
+                                                    : least;
   }
-  return want > least ? want : least;
+  if (!is_gemm_family(base_op(op))) return sk_workspace_bytes(op, M, N, K, nullptr);
+  CallPlan cp, alt;
+  if (plan_call(op, M, N, K, nullptr, &cp)) return 0;
+  return stream_call(op, M, N, K, cp, 0, &alt) ? std::max(cp.need, alt.need) : cp.need;
 }
 
 int sk_gemm_bf16(const sk_bf16* A, int64_t lda, const sk_bf16* W, int64_t ldw, sk_bf16* C, int64_t ldc, int M, int N,

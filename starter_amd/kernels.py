@@ -42,7 +42,7 @@ import torch
 from . import _lib
 from ._lib import (SK_OP_ARGMAX, SK_OP_GATEUP, SK_OP_GEMM, SK_OP_LM_ARGMAX, SK_OP_PRE_GATEUP, SK_OP_PRE_GEMM,
                    SK_OP_PRE_LM_ARGMAX, SK_OP_RESID_GEMM, SK_OP_RMSNORM_GATEUP, SK_OP_RMSNORM_GEMM,
-                   SK_OP_RMSNORM_LM_ARGMAX, SK_PATH_GEMV, SK_PATH_MFMA, SkConfig, check, cfg_ptr, lib)
+                   SK_OP_RMSNORM_LM_ARGMAX, SK_PATH_AUTO, SK_PATH_GEMV, SK_PATH_MFMA, SkConfig, check, cfg_ptr, lib)
 
 BF16 = torch.bfloat16
 
@@ -82,8 +82,9 @@ def _workspace(op: int, M: int, N: int, K: int, cfg: SkConfig | None, device) ->
     every call leaves them at zero again.  Without a configuration it is sized
     for the library's fastest plan, which may split K where the least
     workspace does not allow it."""
-    n = _lib.workspace_bytes(op, M, N, K, cfg) if cfg is not None or op == SK_OP_ARGMAX else \
-        _lib.workspace_bytes_preferred(op, M, N, K)
+    auto = cfg is None or cfg.path == SK_PATH_AUTO
+    n = _lib.workspace_bytes_preferred(op, M, N, K) if auto and op != SK_OP_ARGMAX else \
+        _lib.workspace_bytes(op, M, N, K, cfg)
     return torch.zeros(n, dtype=torch.uint8, device=device) if n else None
 
 
@@ -127,7 +128,12 @@ def _config(config: SkConfig | None, kw: dict) -> SkConfig | None:
 
 
 # ---------------------------------------------------------------------------
-# Functional entry points
+# Functional entry points.  Without ``ws`` a call allocates one only where it
+# cannot run without: at row counts whose fastest plan splits K and whose table
+# plan does not (down at 3-16 rows, o_proj at 17-64), allocating and zeroing a
+# workspace on each call costs more (18.5 against 13.3 us a call) than the plan
+# gains, so there these functions run the table's plan, and round otherwise
+# than the classes below, which hold their workspace.
 # ---------------------------------------------------------------------------
 
 def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, config: SkConfig | None = None,

@@ -250,14 +250,15 @@ def test_preferred_workspace_covers_the_least():
 @pytest.mark.parametrize("N,Kd,M", [(40960, 192, 130), (45001, 640, 177)])
 def test_argmax_of_every_launch_of_a_call(N, Kd, M):
     """Past 128 rows the remainder is a launch of its own, with a plan of its
-    own.  Bound: a logit is one bf16 rounding (2^-9 relative) away from the
-    exact one, so the row's pick may trail the exact best by two."""
+    own.  Bound: a logit is one bf16 rounding (half a unit of 8 significant
+    bits, 2^-8 relative at most) away from the exact one, so the row's pick may
+    trail the exact best by two."""
     g = torch.Generator().manual_seed(N + M)
     w, x = randn_bf16((N, Kd), 0.02, g).to(DEV), randn_bf16((M, Kd), 1.0, g).to(DEV)
     ids, maxv = K.LmArgmax(M, N, Kd, DEV)(x, w)
     exact = x.double() @ w.double().t()
     best = exact.max(-1).values
     picked = exact.gather(1, ids[:, None])[:, 0]
-    step = 2.0 ** -9 * best * 1.01   # (fp32 accumulation: far below)
+    step = 2.0 ** -8 * best * 1.01   # (fp32 accumulation: far below)
     assert bool((best - picked <= 2 * step).all())
     assert bool(((maxv.double() - picked).abs() <= step).all())

@@ -57,7 +57,8 @@ def test_normed_calls_share_a_workspace(N, Kd, M):
     h = xo.double()
     h = h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + 1e-6) * gain.double()
     want = (h @ w.double().t()).float()
-    # bf16 rounding of the norm's two steps and of the output, all relative: 3 * 2^-9 on each term of the sum
+    # three independent bf16 roundings (normed, scaled, output) of at most 2^-8, so 2^-8 / sqrt(3) each in 2-norm:
+    # 2^-8 together, and half of that for margin
     assert ((first.float() - want).norm() / want.norm()).item() < 3 * 2.0 ** -9
     assert not bool(ws[:COUNTERS].any())
     explicit = call(config=_lib.default_config(K.SK_OP_RMSNORM_GEMM, M, N, Kd))
@@ -84,3 +85,21 @@ def test_launches_past_128_rows(M):
             out = torch.full((M, N), float("nan"), dtype=BF16, device=DEV)
             assert_parity(K.gemm(xd, wd, out=out, ws=ws), ref, f"M={M} workspace {n}")
             assert not bool(ws[:512].any())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,Kd,M", [(2560, 9728, 3), (2560, 9728, 16), (2560, 4096, 17), (2560, 4096, 64)])
+def test_the_function_runs_without_a_workspace_and_the_class_with_its_own(N, Kd, M):
+    """Where only the stream plan needs a workspace: the class holds one and
+    takes that plan, the function allocates none and takes the table's, each
+    bit for bit as with that configuration passed explicitly."""
+    g = torch.Generator().manual_seed(N + M)
+    x, w = randn_bf16((M, Kd), 1.0, g).to(DEV), randn_bf16((N, Kd), 0.02, g).to(DEV)
+    mm = K.SkinnyMatmul(M, N, Kd, DEV)
+    selected = _lib.selected_config(K.SK_OP_GEMM, M, N, Kd)
+    assert selected.path == _lib.SK_PATH_STREAM and selected.split > 1 and mm.ws is not None
+    assert torch.equal(mm(x, w), K.gemm(x, w, config=selected))
+    auto = _lib.SkConfig.make(path=_lib.SK_PATH_AUTO)
+    assert torch.equal(mm(x, w), K.SkinnyMatmul(M, N, Kd, DEV, config=auto)(x, w))
+    table = _lib.default_config(K.SK_OP_GEMM, M, N, Kd)
+    assert torch.equal(K.gemm(x, w), K.gemm(x, w, config=table))
