@@ -71,6 +71,7 @@ struct FnInfo {
   size_t spill = 0;
 };
 std::unordered_map<const void*, FnInfo> g_fn;
+std::unordered_map<const void*, size_t> g_lds[64];   // per device: dynamic LDS a kernel is allowed so far
 std::unordered_map<unsigned long long, int> g_occ;
 
 int fn_info(const void* fn, FnInfo* out) {
@@ -85,6 +86,20 @@ int fn_info(const void* fn, FnInfo* out) {
     it = g_fn.emplace(fn, f).first;
   }
   *out = it->second;
+  return SK_OK;
+}
+
+// Allow fn `lds` bytes of dynamic LDS on the current device.  Set when a launch
+// needs more than any before it, not on each launch (the runtime call is host
+// time of every eager call).
+int allow_lds(const void* fn, size_t lds) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return SK_ERR_DEVICE;
+  std::lock_guard<std::mutex> lk(g_mu);
+  size_t& have = g_lds[dev][fn];
+  if (have >= lds) return SK_OK;
+  if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return SK_ERR_CONFIG;
+  have = lds;
   return SK_OK;
 }
 
@@ -855,11 +870,7 @@ int bind_plan(Plan* pl, int num_cu, int* grid) {
   const int tiles_per = cdiv(pl->nrb, *grid / S);
   pl->lds = epi_base(pl->epi) == sk::EPI_ARGMAX ? pl->lds : plan_lds(*pl, 0, tiles_per);
   if (pl->lds > kMaxLds) return SK_ERR_CONFIG;
-  if (pl->lds > 64 * 1024 &&
-      hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)pl->lds) != hipSuccess)
-    return SK_ERR_CONFIG;
-  return SK_OK;
+  return pl->lds > 64 * 1024 ? allow_lds(reinterpret_cast<const void*>(fn), pl->lds) : SK_OK;
 }
 
 // Device address of the current device's copy of `scratch`, looked up once

@@ -9,6 +9,7 @@
 
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <atomic>
 #include <math.h>
 #include <string.h>
 
@@ -852,9 +853,17 @@ template <int QR, bool TREE, bool ROPE>
 int attn_launch(const sk::AttnArgs& a, unsigned grid, hipStream_t stream) {
   constexpr int lds = sk::attn_lds(QR, kAttnWaves);
   const auto fn = &sk::decode_attn_kernel<QR, kAttnWaves, TREE, ROPE>;
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, lds) !=
-      hipSuccess)
-    return SK_ERR_LAUNCH;
+  // (once per device: the runtime call is host time of every eager call)
+  static std::atomic<unsigned long long> allowed{0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return SK_ERR_DEVICE;
+  const unsigned long long bit = dev >= 0 && dev < 64 ? 1ull << dev : 0ull;
+  if (!(allowed.load(std::memory_order_acquire) & bit)) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, lds) !=
+        hipSuccess)
+      return SK_ERR_LAUNCH;
+    allowed.fetch_or(bit, std::memory_order_release);
+  }
   fn<<<dim3(grid), dim3(64 * kAttnWaves), lds, stream>>>(a);
   return attn_launch_status();
 }
