@@ -627,7 +627,9 @@ const StreamEntry kStream[] = {
     {SK_OP_GEMM, 2560, 9728, 65, 128, {5, 4, 4, 40, 4, 0, 4}},      // down 96 rows 21.7 (24.3), 128 23.2 (27.6)
     {SK_OP_GEMM, 2560, 9728, 65, 128, {5, 4, 4, 32, 3, 0, 4}},      // down 96 rows 22.5, 128 24.5
     // residual producers (tiles of whole 16-column groups)
-    {SK_OP_RESID_GEMM, 2560, 4096, 17, 64, {5, 4, 2, 32, 3, 0, 2}},     // o_proj 32 rows 9.8 (10.1), 64 12.5 (14.0)
+    // (o_proj at 41-48 rows: the table's three row groups of 16 take 11.4 us, this 11.6-11.8)
+    {SK_OP_RESID_GEMM, 2560, 4096, 17, 40, {5, 4, 2, 32, 3, 0, 2}},     // o_proj 32 rows 9.8 (10.1)
+    {SK_OP_RESID_GEMM, 2560, 4096, 49, 64, {5, 4, 2, 32, 3, 0, 2}},     // o_proj 64 rows 12.5 (14.0)
     {SK_OP_RESID_GEMM, 2560, 4096, 97, 128, {5, 4, 4, 32, 3, 0, 4}},    // o_proj 128 rows 17.9 (20.7)
     {SK_OP_RESID_GEMM, 2560, 9728, 3, 16, {5, 4, 2, 32, 3, 0, 1}},      // down 8 rows 12.9 (14.8), 16 13.3 (15.2)
     {SK_OP_RESID_GEMM, 2560, 9728, 17, 64, {5, 4, 2, 32, 3, 0, 2}},     // down 32 rows 15.7 (20.0), 64 21.1 (28.2)

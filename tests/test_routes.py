@@ -22,7 +22,7 @@ RANGES = [
     (GEMM, 2560, 4096, ((17, 64), (97, 128))),
     (GEMM, 2560, 9728, ((3, 128),)),
     (GATEUP, 9728, 2560, ((17, 128),)),
-    (RESID, 2560, 4096, ((17, 64), (97, 128))),
+    (RESID, 2560, 4096, ((17, 40), (49, 64), (97, 128))),
     (RESID, 2560, 9728, ((3, 128),)),
     (GEMM, 151936, 2560, ((33, 128),)),
     (ARGMAX, 151936, 2560, ((49, 128),)),
