@@ -83,8 +83,13 @@ __device__ __forceinline__ i32x4 buf_of(const void* p, int bytes) {
 }
 
 // 16 bytes per lane from descriptor r at byte voff + soff into LDS at lds_off
-// + 16 * lane.  No register is written, so the compiler need not track it;
-// the caller waits on vmcnt.
+// + 16 * lane.  No vector register is written, so the compiler need not track
+// it; the caller waits on vmcnt.  m0 is overwritten and cannot be declared: it
+// is a reserved register, which the compiler warns about in a clobber list and
+// does not preserve.  It never allocates m0 either, so this is safe as long as a
+// kernel has no instruction of the compiler's own that reads it (indexed
+// register access, messages, LDS-direct builtins); tests/test_build_tiers.py
+// checks the assembly.
 template <bool STREAM>
 __device__ __forceinline__ void load_lds16(uint32_t lds_off, int voff, i32x4 r, int soff) {
   if constexpr (STREAM)

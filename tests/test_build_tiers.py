@@ -9,6 +9,9 @@ planner in the built library enforces the committed table.
 
 from __future__ import annotations
 
+import re
+import subprocess
+
 import pytest
 
 import starter_amd.build as B
@@ -137,3 +140,20 @@ def test_remarks_report_spills_and_reject_private_arrays():
     stack = _remarks(("_ZN2sk11wide2_entryILi8ELi6ELi1EEEvNS_4ArgsE", 208, 0))
     with pytest.raises(RuntimeError, match="private memory"):
         B._run(_fake_hipcc(stack))
+
+
+@pytest.mark.parametrize("unit,defs", [("sk_attn.hip", []), ("sk_inst_stream.hip", ["-DSK_EPI=2"])])
+def test_only_the_direct_lds_loads_use_m0(unit, defs, tmp_path):
+    """The inline assembly of the direct loads overwrites m0, which a clobber
+    list cannot declare: no instruction outside those blocks may use it."""
+    out = tmp_path / "unit.s"
+    subprocess.run([B.HIPCC, *B.COMMON, *defs, "--cuda-device-only", "-S", str(B.CSRC / unit), "-o", str(out)],
+                   check=True, capture_output=True)
+    inside, loads, stray = False, 0, []
+    for line in out.read_text().splitlines():
+        if "#ASMSTART" in line or "#ASMEND" in line:
+            inside = "#ASMSTART" in line
+        elif re.search(r"\bm0\b", line.split(";")[0]):
+            loads += inside
+            stray += [] if inside else [line]
+    assert loads > 0 and not stray, stray[:5]
