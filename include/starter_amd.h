@@ -26,8 +26,10 @@
  * zero-filled (outside graph capture).  Its first bytes hold arrival counters
  * that let the last workgroup of a tile finish a split-K sum or an argmax in
  * the same kernel; every call leaves them at zero again, so the workspace is
- * reused without clearing.  Calls that share one workspace must not overlap
- * (same stream, or ordered by events).
+ * reused without clearing.  One workspace serves calls of its op and shape
+ * without a configuration and with sk_default_config's, whatever their strides.
+ * Calls that share one workspace must not overlap (same stream, or ordered by
+ * events).
  */
 #ifndef STARTER_AMD_H
 #define STARTER_AMD_H
@@ -214,9 +216,12 @@ int sk_gemm_bf16(const sk_bf16* A, int64_t lda, const sk_bf16* W, int64_t ldw,
 /* sk_gemm_bf16 without a workspace argument: no counterpart in the reference.
  * For callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
- * arguments, kernels and results as sk_gemm_bf16; the split-K arrival
- * counters and partials live in a static device array of
- * SK_NOALLOC_SCRATCH_BYTES (4 MiB) per GPU, held until the process ends.  The
+ * arguments as sk_gemm_bf16, and the kernels and results of that call with a
+ * workspace of sk_workspace_bytes (with more, sk_gemm_bf16 may take another
+ * plan; this one does not, so a call whose least workspace is none touches no
+ * shared scratch).  The split-K arrival counters and partials live in a static
+ * device array of SK_NOALLOC_SCRATCH_BYTES (4 MiB) per GPU, held until the
+ * process ends.  The
  * call allocates nothing (no hipMalloc/hipFree, no allocating library call);
  * a plan that needs more scratch than that returns SK_ERR_SCRATCH before
  * anything is enqueued.  A split-K call first clears the counters it uses

@@ -464,7 +464,8 @@ size_t plan_workspace(int op, int M, int N, const Plan& pl) {
   return 0;
 }
 
-// Offline-tuned launch table for the Qwen3-4B decode shapes (the reference
+// Offline-tuned launch table for the Qwen3-4B decode shapes, what a call
+// without a configuration runs where no stream plan (kStream) takes its place (the reference
 // picks a Triton config per shape at warmup: engine/kernels/gemm.py:516-660).
 // Each entry is the fastest configuration measured on one MI355X for that
 // shape at that row count, timed as graph replays of back-to-back launches
@@ -604,9 +605,9 @@ const Tuned kTuned[] = {
 //    (about 2.5 us).  Their least workspace (sk_workspace_bytes) allows three
 //    splits of 32-row tiles or none; sk_workspace_bytes_preferred covers the
 //    first entry.
-//  * qkv and o_proj up to 16 rows and gate_up up to 16 stay on the ring path
-//    where that measured within 2%; qkv at 49-64 rows runs 128-column units
-//    (13.4 us with 64-column ones).
+//  * qkv at one row, o_proj and gate_up up to 16, down up to two and o_proj at
+//    65-96 have no entry: the table's plan measured faster or within 2%.  qkv at
+//    49-64 rows runs 128-column units (13.4 us with 64-column ones).
 struct StreamEntry {
   int op, N, K, m_lo, m_hi;
   sk_config cfg;   // {path, waves, ku = unit columns / 32, tile rows, split, 0, waves per K group}

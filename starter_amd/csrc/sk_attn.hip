@@ -280,10 +280,10 @@ __device__ __forceinline__ void load_agent_vec(__amdgpu_buffer_rsrc_t r, int off
 // ranges of the planned length left most workgroups of a shorter sequence
 // without keys (one sequence, 2000 of 4096 planned keys: half of them, 14.2 us
 // against 9.9; 4 of 4000 of 8192: 19.8 against 14.4).  A sequence of at most
-// WHOLE_GRAINS keeps one range: another block of 16 keys per wave costs about
-// 0.9 us, publishing and merging ranges 2-3 us (one query row, 300 keys: 7.1 us
-// in one range, 7.3 in three; 16 sequences of 300: 8.7 and 9.9; at 500 keys
-// 9.2 in one or two, 8.1 in four).
+// WHOLE_GRAINS keeps one range: another block of 16 keys per wave costs less
+// than 1 us, publishing and merging ranges about 1.5 (one query row, 300 keys:
+// 7.3 us in one range, 8.1 in three; 16 sequences of 300: 9.4 and 10.4; past it,
+// one of 500 keys 9.8 in one range, 8.7 in four; 16 of up to 500 10.6 and 10.3).
 constexpr int KEY_GRAIN = 64, WHOLE_GRAINS = 6;
 struct KeyRange {
   int pos, len;        // the sequence's position and keys
@@ -355,10 +355,12 @@ __global__ void __launch_bounds__(64 * ATTN_WAVES, 4) decode_attn_kernel(AttnArg
   // fragments are in registers, so four to eight loads of a wave are always in
   // flight, and nothing is staged in registers: 119 of them at most, two
   // workgroups per CU (blocks staged in registers took 180 and one: 64
-  // sequences of up to 200 keys 13.7 us, now 11.5; 5 x 8 tree rows 28.3 us,
-  // now 17.2).  Long contexts are bound by memory (2 x 32000 keys: 42 us, 5.8
-  // TB/s at the mean of both lengths), short ones by the chain of round trips
-  // position, projection row, keys, merge.
+  // sequences of up to 200 keys 14.4 us, now 11.5; 5 x 8 tree rows of up to 1000
+  // 16.4 us, now 13.1).  A second slot per wave is slower (16 sequences of up
+  // to 500 keys 10.6 -> 10.9 us, 64 of up to 200 12.0 -> 15.6): it takes the CU's
+  // second workgroup, and more requests in flight per wave bring nothing.  Long
+  // contexts are bound by memory (2 x 32000 keys 44.7 us, 5.9 TB/s), short ones
+  // by the chain of round trips position, projection row, keys, merge.
   //  * Scores: S^T[key][row] = K[16 keys, 128] . Q^T by four MFMAs with K as
   //    the A operand (lane l: key l%16, dims 32s + 8*(l/16)).  Chunk c (16
   //    bytes) of key r lies at position c ^ r of its row, so the 16 keys of a
@@ -746,9 +748,9 @@ int attn_plan(int B, int HQ, int HKV, int D, int R, int cap, int max_len, int ns
   if (rows > kAttnMaxRows) return SK_ERR_SHAPE;
   // Query rows per workgroup: up to 16, the columns of the MFMA tiles (the
   // per-lane state does not grow with them); more rows take several row
-  // blocks, each streaming the keys once more.  The smaller instances keep
-  // less LDS and epilogue work (B = 16, 1088 keys, R = 2: 17.1 us with 8
-  // rows, 17.8 us with 16).
+  // blocks, each streaming the keys once more.  The smaller instances have
+  // less prologue and epilogue work (one row, 300 keys: 7.3 us with 4 rows, 7.5
+  // with 8; 16 sequences of up to 1088 keys, R = 2: 18.0 with 8, 18.1 with 16).
   p->QR = rows <= 4 ? 4 : rows <= 8 ? 8 : 16;
   p->NRB = cdiv(rows, p->QR);
   const int work = max_len > 0 && max_len < cap ? max_len : cap;
