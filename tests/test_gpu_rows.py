@@ -62,7 +62,7 @@ def test_swiglu_of_few_rows_is_no_slower_in_16_byte_accesses(M):
     stride selects) where launch and latency decide: a thread must not work
     through several rows while most of the chip is idle (that took 1.2 to 1.8
     times as long here)."""
-    I, reps = 9728, 10
+    I, reps = 9728, 200   # (one replay of 0.5 ms: its launch, which may vary by 5 us, does not count)
     gu = torch.randn(M, 2 * I, device=DEV).to(BF16)
 
     def best(out):
