@@ -262,3 +262,22 @@ def test_argmax_of_every_launch_of_a_call(N, Kd, M):
     step = 2.0 ** -8 * best * 1.01   # (fp32 accumulation: far below)
     assert bool((best - picked <= 2 * step).all())
     assert bool(((maxv.double() - picked).abs() <= step).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,Kd,grid,M", [(2577, 2048, 16, 100), (700, 4096, 44, 33), (3000, 320, 60, 64), (4100, 64, 256, 128),
+                                         (1500, 2048, 9, 1)])
+def test_stream_persistent_tiles_of_4_kb_strides(N, Kd, grid, M):
+    """Row strides that are multiples of 4 KB: the workgroups start their tiles
+    at units of their own, and a tile's first and last units wrap around."""
+    g = torch.Generator().manual_seed(N + Kd + M)
+    w, x = randn_bf16((N, Kd), 0.02, g), randn_bf16((M, Kd), 1.0, g)
+    ld = (Kd + 2047) // 2048 * 2048
+    wide = torch.full((N, ld), float("nan"), dtype=BF16, device=DEV)
+    wide[:, :Kd] = w.to(DEV)
+    xd, wd = x.to(DEV), wide[:, :Kd]
+    out = K.gemm(xd, wd, config=tiles(grid))
+    assert_parity(out, from_bits(oracle.gemm(bits(x), bits(w))), f"N={N} K={Kd} grid={grid} M={M}")
+    ids, maxv = K.lm_argmax(xd, wd, config=tiles(grid))
+    best = out.float().max(-1).values
+    assert torch.equal(maxv, best) and torch.equal(ids, (out.float() == best[:, None]).float().argmax(-1))
