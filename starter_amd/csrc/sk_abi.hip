@@ -657,6 +657,26 @@ const StreamEntry* stream_lookup(int op, int M, int N, int K, int n) {
   return nullptr;
 }
 
+// Whether the persistent tiles are the faster plan of M rows beside the general
+// one.  A workgroup's slabs rarely fill its last tile, and a tile costs the same
+// time with one slab as with all: `fill` is the share of the tiles' rows that
+// exist.  The one general plan that comes near is the ring path with one K split
+// and seven or more waves of 256 columns (K 1792-2048 up to 64 rows, up to 3072 at
+// 33-48).  us, that plan against tiles: 41024 x 2048 (fill 0.50) logits 64 rows
+// 38.1, 42.1, argmax 49 37.8, 44.4; 49152 x 2048 (0.60) argmax 49 41.9, 48.0;
+// 57344 x 2048 (0.70) logits 64 49.5, 46.4; 41024 x 2560 (0.50) 33 rows 41.6, 53.2;
+// 49152 x 3072 (0.60) 48 rows 54.2, 62.2; 57344 x 3072 (0.70) 48 rows 61.8, 64.9;
+// 65536 x 2560 (0.80) 48 rows 74.9, 60.9; 131072 x 2560 (0.80) 33 rows 110, 123;
+// 81920 x 2560 (1.00) 33 rows 70.9, 69.6.  Other general plans are slower at any
+// fill (41024 x 2304, 64 rows, two K splits: 157, 48.2; 41024 x 1280: 38.7, 31.0).
+bool tiles_pay(int M, int N, const Plan& general) {
+  if (general.cfg.path != SK_PATH_MFMA_LDS || general.cfg.split != 1 || general.cfg.waves < 7) return true;
+  constexpr int per_tile = sk::kTilesRows / 16;
+  const long slabs = cdiv(N, 16), tiles = cdiv(cdiv((int)slabs, 256), per_tile);
+  const long fill = 100 * slabs / (256 * tiles * per_tile);
+  return fill >= (M <= 40 ? 90 : M <= 48 ? 75 : 65);
+}
+
 // Counter bytes of the widest stream plan of op/N/K, whatever its rows (0: none
 // has counters).
 size_t stream_counters(int op, int N, int K) {
@@ -1020,6 +1040,7 @@ bool stream_call(int op, int M, int N, int K, const CallPlan& cp, int n, CallPla
   bool any = false;
   for (int i = 0; i < cp.nplans; ++i) {
     if (const StreamEntry* e = stream_lookup(bop, cp.chunk_rows[i], N, K, n)) {
+      if (e->cfg.grid > 0 && !tiles_pay(cp.chunk_rows[i], N, cp.plans[i])) continue;
       Plan pl;
       if (plan_shape_impl(bop, cp.chunk_rows[i], N, K, e->cfg, false, &pl) == SK_OK) {
         pl.norm = cp.plans[i].norm;

@@ -28,6 +28,15 @@ RANGES = [
     (ARGMAX, 151936, 2560, ((49, 128),)),
     (GEMM, 40960, 320, ((33, 128),)),
     (GEMM, 40959, 320, ()),            # fewer rows than a tile for every CU
+    # beside a ring plan of seven waves and more: by the share of the tiles' rows that exist
+    (GEMM, 41024, 2048, ()),           # 0.50
+    (ARGMAX, 41024, 2048, ()),
+    (GEMM, 41024, 1536, ((33, 128),)),     # six waves
+    (GEMM, 41024, 2560, ((49, 128),)),     # ten waves, but two K splits past 48 rows
+    (GEMM, 57344, 2048, ((49, 128),)),     # 0.70
+    (ARGMAX, 57344, 2048, ((49, 128),)),
+    (GEMM, 65536, 2048, ((41, 128),)),     # 0.80
+    (GEMM, 81920, 2048, ((33, 128),)),     # 1.00
     (GEMM, 40960, 352, ()),            # K not whole 64-column units
     (GEMM, 777, 2560, ()),
 ]
