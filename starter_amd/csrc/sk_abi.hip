@@ -1582,8 +1582,11 @@ int sk_swiglu_bf16(const sk_bf16* gu, int64_t ld_gu, sk_bf16* out, int64_t ld_ou
   int st = device_info(&num_cu);
   if (st) return st;
   if (I % 8 == 0 && ((ld_gu | ld_out) & 7) == 0 && aligned16(gu) && aligned16(out)) {
-    sk::swiglu_vec_kernel<<<dim3((unsigned)cdiv(I, 8 * 256), (unsigned)(M < 65535 ? M : 65535)), dim3(256), 0,
-                            stream>>>(gu, ld_gu, out, ld_out, M, I);
+    int shift = 0;   // threads per row: a power of two that covers it, at most the workgroup
+    while (shift < 8 && (8 << shift) < I) ++shift;
+    const int rb = cdiv(M, 256 >> shift);
+    sk::swiglu_vec_kernel<<<dim3((unsigned)cdiv(I, 8 << shift), (unsigned)(rb < 65535 ? rb : 65535)), dim3(256), 0,
+                            stream>>>(gu, ld_gu, out, ld_out, M, I, shift);
     return launch_status();
   }
   const long total = (long)M * I;

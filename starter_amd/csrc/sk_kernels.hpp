@@ -1594,17 +1594,21 @@ __global__ void __launch_bounds__(256) clear_words_kernel(unsigned* __restrict__
 
 // Unfused SwiGLU over gu = [g | u] (engine/kernels/swiglu.py:14-24), eight
 // columns per thread: rows of 8-column multiples whose base and strides are
-// 16-byte aligned.  Workgroup (column block, row).  Bound by memory from some
+// 16-byte aligned.  Workgroup (column block, rows): 1 << row_shift threads per
+// row, so that narrow rows share one (16384 rows x 64 in a workgroup each took
+// 11.3 us, so 5).  Bound by memory from some
 // hundred rows on: 16384 rows x 9728 (956 MB) 175 us, 5.5 TB/s, where 2-byte
 // accesses take 280; below, by the launch and one thread's chain of loads and
 // exponentials.  So a thread takes one row: with four rows each (and a quarter
 // of the workgroups) the chain took 4.7 us at 4-64 rows x 9728 where one row
 // takes 2.7-3.2 and 2-byte accesses 2.6-4.0, and 180 us at 16384.
 __global__ void __launch_bounds__(256) swiglu_vec_kernel(const uint16_t* __restrict__ gu, int64_t ld_gu,
-                                                         uint16_t* __restrict__ out, int64_t ld_out, int M, int I) {
-  const int i = 8 * (blockIdx.x * 256 + threadIdx.x);
+                                                         uint16_t* __restrict__ out, int64_t ld_out, int M, int I,
+                                                         int row_shift) {
+  const int i = 8 * ((blockIdx.x << row_shift) + (threadIdx.x & ((1 << row_shift) - 1)));
   if (i >= I) return;
-  for (int m = blockIdx.y; m < M; m += gridDim.y) {
+  const int rows = 256 >> row_shift;   // of a workgroup
+  for (int m = blockIdx.y * rows + (threadIdx.x >> row_shift); m < M; m += gridDim.y * rows) {
     const uint16_t* row = gu + (int64_t)m * ld_gu + i;
     const u32x4 g = ld16_stream(row), u = ld16_stream(row + I);
     u32x4 y;

@@ -50,9 +50,12 @@ def test_swiglu_forms_equal_the_oracle(M, I):
             assert (out[oby:].view(M, I + opad)[:, I:] == 7.0).all()
 
 
-def test_swiglu_of_more_rows_than_the_grid_has():
-    g = torch.Generator().manual_seed(5)
-    gu = randn_bf16((65535 + 9, 16), 3.0, g)
+@pytest.mark.parametrize("M,I", [(65535 + 9, 2048), (700, 8), (513, 16), (129, 72), (3, 1032), (1000, 1016)])
+def test_swiglu_of_every_row_packing(M, I):
+    """1 to 256 threads per row, part of them idle, a last workgroup with fewer
+    rows, and more rows than the grid has."""
+    g = torch.Generator().manual_seed(M + I)
+    gu = randn_bf16((M, 2 * I), 3.0, g)
     assert np.array_equal(bits(K.swiglu(gu.to(DEV))), oracle.swiglu(bits(gu)))
 
 
