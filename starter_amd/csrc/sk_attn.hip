@@ -831,7 +831,12 @@ int sk_qk_norm_rope_cache_bf16(const sk_bf16* qkv, int64_t ld_qkv, const sk_bf16
   a.HKV = HKV;
   a.cap = cap;
   a.eps = eps;
-  if (aligned16(qkv) && (ld_qkv & 7) == 0 && aligned16(q_norm_w) && aligned16(k_norm_w) && aligned16(cos) &&
+  // 16-byte accesses from about a thousand heads on: with fewer, one lane's
+  // chain of eight elements costs more than the loads it saves (32 + 2 x 8 heads,
+  // us, one element per lane against eight: 8 rows 2.54, 2.63; 24 2.64, 2.68; 32
+  // 2.77, 2.72; 128 3.75, 3.39).  Both give the same bits.
+  const bool many = (int64_t)B * T * (HQ + 2 * HKV) >= 1024;
+  if (many && aligned16(qkv) && (ld_qkv & 7) == 0 && aligned16(q_norm_w) && aligned16(k_norm_w) && aligned16(cos) &&
       aligned16(sin) && aligned16(q_out) && aligned16(k_cache) && aligned16(v_cache)) {
     sk::qk_norm_rope_vec_kernel<<<dim3((unsigned)(B * T), (unsigned)cdiv(HQ + 2 * HKV, 16)), dim3(256), 0, stream>>>(a);
     return attn_launch_status();

@@ -95,7 +95,9 @@ def test_swiglu_of_few_rows_is_no_slower_in_16_byte_accesses(M):
 
 @pytest.mark.parametrize("B,T,HQ,HKV,cap,tree", [
     (2, 33, 32, 8, 128, False), (3, 1, 4, 2, 64, False), (1, 5, 5, 1, 20, True), (2, 8, 8, 2, 40, True),
-    (1, 300, 3, 3, 256, False)])   # the last: rows past the cache and past the table are skipped
+    (1, 300, 3, 3, 256, False),   # rows past the cache and past the table are skipped
+    (50, 8, 5, 1, 300, True), (4, 1, 200, 28, 64, False), (1, 342, 1, 1, 400, True),   # from 1024 heads on 16-byte rows
+    (1, 341, 1, 1, 400, False)])                                                      # the most that take the other kernel
 def test_rope_vector_rows_equal_scalar_rows(B, T, HQ, HKV, cap, tree):
     g = torch.Generator().manual_seed(B * T)
     W = (HQ + 2 * HKV) * D
