@@ -1020,12 +1020,21 @@ int plan_call(int op, int M, int N, int K, const sk_config* cfg, CallPlan* cp) {
     if (uses_counters(op, cp->plans[i])) cp->counters = std::max(cp->counters, plan_tickets(op, cp->plans[i]));
   // The remainder of a call without a configuration has a plan of its own; the
   // default configuration passed explicitly shares its workspace all the same.
-  CallPlan def;
-  if (cp->nplans == 2 && !cp->fused && cfg && cfg->path != SK_PATH_AUTO &&
-      plan_call(op, M, N, K, nullptr, &def) == SK_OK && !def.fused)
-    cp->counters = std::max(cp->counters, def.counters);
+  if (cp->nplans == 2 && !cp->fused && cfg && cfg->path != SK_PATH_AUTO) {
+    CallPlan def;
+    if (plan_call(op, M, N, K, nullptr, &def) == SK_OK && !def.fused)
+      cp->counters = std::max(cp->counters, def.counters);
+  }
   lay_out(op, M, N, K, cp);
   return SK_OK;
+}
+
+// Whether any launch of cp has an n-th stream entry (most calls of eager code
+// have none: they make no further plans).
+bool has_stream(int op, int N, int K, const CallPlan& cp, int n) {
+  for (int i = 0; i < cp.nplans && !cp.fused; ++i)
+    if (stream_lookup(base_op(op), cp.chunk_rows[i], N, K, n)) return true;
+  return false;
 }
 
 // The call with stream-path plans in place of cp's, taking the n-th entry of
@@ -1057,12 +1066,14 @@ bool stream_call(int op, int M, int N, int K, const CallPlan& cp, int n, CallPla
 // cp, or the first stream entry's that fit them.  False when not even cp fits.
 bool select_call(int op, int M, int N, int K, size_t avail, CallPlan* cp) {
   if (cp->need > avail) return false;
-  CallPlan alt;
-  for (int n = 0; stream_call(op, M, N, K, *cp, n, &alt); ++n)
+  for (int n = 0; has_stream(op, N, K, *cp, n); ++n) {
+    CallPlan alt;
+    if (!stream_call(op, M, N, K, *cp, n, &alt)) break;
     if (alt.need <= avail) {
       *cp = alt;
       break;
     }
+  }
   return true;
 }
 
@@ -1475,8 +1486,10 @@ size_t sk_workspace_bytes_preferred(int op, int M, int N, int K) {
                                                     : least;
   }
   if (!is_gemm_family(base_op(op))) return sk_workspace_bytes(op, M, N, K, nullptr);
-  CallPlan cp, alt;
+  CallPlan cp;
   if (plan_call(op, M, N, K, nullptr, &cp)) return 0;
+  if (!has_stream(op, N, K, cp, 0)) return cp.need;
+  CallPlan alt;
   return stream_call(op, M, N, K, cp, 0, &alt) ? std::max(cp.need, alt.need) : cp.need;
 }
 
