@@ -1596,7 +1596,7 @@ __global__ void __launch_bounds__(256) clear_words_kernel(unsigned* __restrict__
 // columns per thread: rows of 8-column multiples whose base and strides are
 // 16-byte aligned.  Workgroup (column block, rows): 1 << row_shift threads per
 // row, so that narrow rows share one (16384 rows x 64 in a workgroup each took
-// 11.3 us, so 5).  Bound by memory from some
+// 11.3 us, so 3.3).  Bound by memory from some
 // hundred rows on: 16384 rows x 9728 (956 MB) 175 us, 5.5 TB/s, where 2-byte
 // accesses take 280; below, by the launch and one thread's chain of loads and
 // exponentials.  So a thread takes one row: with four rows each (and a quarter
